@@ -190,13 +190,14 @@ int64_t qp_prefill_i8_workspace_size(const qp_paged_cache *cache, const qp_prefi
 
 /*
  * One attention step of a batch over the paged cache, routed on the device with no host synchronisation:
- *   - every sequence with 1..QP_DECODE_MAX_QUERY query tokens whose rows fit the segment buffers goes to the split-KV
- *     decode (one workgroup per segment holding the GQA group's rows) and the log-sum-exp merge;
+ *   - every sequence with 1..QP_DECODE_MAX_QUERY query tokens goes to the split-KV decode (one workgroup per segment
+ *     holding the GQA group's rows) and the log-sum-exp merge; where the batch's short sequences can have more rows
+ *     than the segment buffers, the partials of all of them are kept in the workspace instead;
  *   - every other sequence (prefill chunks) goes to the MFMA prefill kernel, or its query-slice path.
  * A batch of short sequences only (max_query_len <= QP_DECODE_MAX_QUERY, num_tokens <= segm_rows) is decode + merge
  * with partial rows at the tokens' own indices and needs no workspace, so it can be recorded in a HIP graph. A mixed
- * batch packs its short sequences' rows into the segment buffers through a route table in the workspace. With
- * rht_signs, q is unrotated (rotated to (q D) H as it loads) and the output is rotated back, (o H D) * rht_out_scale,
+ * batch packs its short sequences' rows into the segment buffers (or the workspace) through a route table in the
+ * workspace. With rht_signs, q is unrotated (rotated to (q D) H as it loads) and the output is rotated back, (o H D) * rht_out_scale,
  * inside the kernels: the call is the whole of unified_attention_int4.
  * Replaces the stock unified_attention_int4 with the reference's router around it (int4_kv.py:294-329: the decode /
  * MTP rows as a split-KV sub-batch, long chunks to the prefill path, single_rht before and after, :307-329).

@@ -293,3 +293,27 @@ def test_drop_in_attention_in_a_hip_graph(device):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), step
+
+
+@pytest.mark.parametrize("fmt,nq,nkv,hs,T", [("int4", NQ, NKV, 256, 1), ("int8", NQ, NKV, 256, 2), ("int4", 16, 4, 128, 4),
+                                             ("int4", 16, 2, 64, 3), ("int4", 16, 2, 512, 4), ("int8", 32, 2, 256, 4)])
+def test_decode_batch_beyond_the_segment_buffers(device, fmt, nq, nkv, hs, T):
+    """A batch of short sequences with more rows than the segment buffers (here 3) keeps its partials in the
+    workspace: the same kernels on the same segments, so the same bits as with buffers that hold every row (the last
+    shape has more query rows per KV head than two row tiles and is routed)."""
+    import torch
+    seqs = [(T, 2100), (1, 1), (T, 700), (max(1, T - 1), 4097), (1, 33)]
+    lens, qlens = [n for _, n in seqs], [t for t, _ in seqs]
+    views, table, _ = _stored_cache(device, fmt, lens, 580 + hs, nkv=nkv, hs=hs)
+    q = torch.randn((sum(qlens), nq, hs), device=device, dtype=torch.bfloat16)
+    cu = i32(np.concatenate(([0], np.cumsum(qlens))), device)
+    got = []
+    for rows in (3, 32):
+        out = torch.full_like(q, float("nan"))
+        segm = _segm(device, rows, 16, nq=nq, hs=hs)
+        _call(views, q, out, cu, i32(lens, device), i32(table, device), max(qlens), max(lens), segm, 16, hs=hs)
+        torch.cuda.synchronize()
+        got.append(out)
+        if rows == 3:
+            assert torch.isnan(segm[0]).all() and torch.isnan(segm[1]).all()
+    assert torch.equal(got[0], got[1]) and torch.isfinite(got[0]).all()

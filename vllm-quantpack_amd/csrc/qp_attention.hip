@@ -6,7 +6,8 @@
 // its FlashAttention prefill, rotating q before and the output after (single_rht, :307-329). Here the split is a
 // route table written by one small kernel, which both kernels read, so the step has no host synchronisation:
 //   * short sequences (1..QP_DECODE_MAX_QUERY query tokens) get consecutive rows of the caller's split-KV segment
-//     buffers while they last; the decode kernel serves them in token groups and the merge writes their output;
+//     buffers, or of the workspace when the batch can have more such rows than the buffers; the decode kernel serves
+//     them in token groups and the merge writes their output;
 //   * every other sequence takes the MFMA prefill kernel (or its query-slice path), which skips the short ones.
 // A batch with short sequences only keeps the tokens' own rows and no table, so it needs no workspace and can be
 // recorded in a HIP graph. The randomized Hadamard rotation is fused: the kernels rotate each query row as it loads
@@ -17,8 +18,7 @@
 
 namespace qp {
 
-// One workgroup. route_row[i]: first segment-buffer row of short sequence i, -1 for the others (and for short ones
-// past the buffer's rows_cap rows, which the prefill then serves). row_tok / row_seq[r]: token and sequence of row r,
+// One workgroup. route_row[i]: first segment-buffer row of short sequence i, -1 for the others. row_tok / row_seq[r]: token and sequence of row r,
 // -1 / 0 for unused rows.
 __global__ __launch_bounds__(256) void route_kernel(const int32_t *cu_q, int num_seqs, int rows_cap,
                                                     int32_t *route_row, int32_t *row_tok, int32_t *row_seq) {
@@ -69,12 +69,56 @@ struct AttentionPlan {
   bool plain_decode;  // short sequences only: decode + merge on the tokens' own rows
   bool routed;        // a route table splits the batch between decode and prefill
   int rows_cap;       // segment-buffer rows the route table hands out
-  int64_t off_route, off_tok, off_seq, off_prefill, total;
+  int64_t off_route, off_tok, off_seq, off_segm, off_prefill, total;
+  int64_t segm_rows;  // rows of split-KV partials in the workspace (0: the caller's segment buffers hold them)
   qp_prefill_args prefill;
   qp_decode_args decode;
 };
 
 int64_t up256(int64_t x) { return (x + 255) / 256 * 256; }
+
+// Split-KV partials in the workspace instead of the caller's segment buffers: [rows, heads, segments, head size] rows,
+// then the maxima and the sums, fp32, each part 256-byte aligned.
+int64_t segm_bytes(int64_t triples, int hs) { return up256(4 * triples * hs) + 2 * up256(4 * triples); }
+
+void segm_in_workspace(AttentionPlan &P, const qp_paged_cache *cache, uint8_t *ws) {
+  const int hs = cache->head_size;
+  qp_decode_args &d = P.decode;
+  const int64_t triples = P.segm_rows * d.num_q_heads * d.num_segments;
+  d.segm_output = reinterpret_cast<float *>(ws + P.off_segm);
+  d.segm_output_stride[2] = hs;
+  d.segm_output_stride[1] = (int64_t)d.num_segments * hs;
+  d.segm_output_stride[0] = (int64_t)d.num_q_heads * d.segm_output_stride[1];
+  d.segm_max = reinterpret_cast<float *>(ws + P.off_segm + up256(4 * triples * hs));
+  d.segm_expsum = reinterpret_cast<float *>(ws + P.off_segm + up256(4 * triples * hs) + up256(4 * triples));
+  d.segm_stat_stride[1] = d.num_segments;
+  d.segm_stat_stride[0] = (int64_t)d.num_q_heads * d.num_segments;
+  d.segm_rows = (int32_t)P.segm_rows;
+}
+
+// The merge of d's partials into a's output, with the inverse rotation when a asks for one.
+qp_merge_args merge_of(const qp_decode_args &d, const qp_attention_args *a, int hs) {
+  qp_merge_args m = {};
+  m.segm_output = d.segm_output;
+  for (int i = 0; i < 3; ++i) m.segm_output_stride[i] = d.segm_output_stride[i];
+  m.segm_max = d.segm_max;
+  m.segm_expsum = d.segm_expsum;
+  m.segm_stat_stride[0] = d.segm_stat_stride[0];
+  m.segm_stat_stride[1] = d.segm_stat_stride[1];
+  m.cu_seqlens_q = a->cu_seqlens_q;
+  m.seqused_k = a->seqused_k;
+  m.num_seqs = a->num_seqs;
+  m.num_tokens = a->num_tokens;
+  m.num_q_heads = a->num_q_heads;
+  m.head_size = hs;
+  m.num_segments = d.num_segments;
+  m.out = a->out;
+  m.out_stride[0] = a->out_stride[0];
+  m.out_stride[1] = a->out_stride[1];
+  m.rht_signs = a->rht_signs;
+  m.rht_out_scale = a->rht_out_scale;
+  return m;
+}
 
 AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_args *a) {
   AttentionPlan P = {};
@@ -84,10 +128,16 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
   const bool decode_shape =
       segm && (hs == 64 || hs == 128 || hs == 256 || hs == 512) && G >= 1 && G <= 32 && (hs != 512 || G <= 16);
   P.plain_decode = decode_shape && a->max_query_len >= 1 && a->max_query_len <= QP_DECODE_MAX_QUERY &&
-                   a->max_query_len * G <= 32 && a->num_tokens <= a->segm_rows;
+                   a->max_query_len * G <= 32;
   P.routed = decode_shape && !P.plain_decode;
+  // Rows of partials the batch's short sequences can have. The caller's segment buffers hold them when they have that
+  // many rows; otherwise the partials go to the workspace, so every short sequence takes the split-KV kernel (an
+  // engine that allocates 128 / KV heads rows sends larger batches than that: 64 sequences over up to 8192 keys at 32
+  // q / 8 KV heads took 280 us with the 48 past the buffers' 16 rows on the prefill kernel, 76 us here).
   const int64_t cap = (int64_t)QP_DECODE_MAX_QUERY * a->num_seqs;
-  P.rows_cap = P.routed ? (int)(a->segm_rows < cap ? a->segm_rows : cap) : 0;
+  const int64_t rows = a->num_tokens < cap ? a->num_tokens : cap;
+  P.rows_cap = P.routed ? (int)rows : 0;
+  P.segm_rows = decode_shape && rows > a->segm_rows ? rows : 0;
 
   qp_decode_args &d = P.decode;
   d.query = a->query;
@@ -111,6 +161,11 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
   d.segm_stat_stride[1] = a->segm_stat_stride[1];
   d.segm_rows = a->segm_rows;
   d.query_signs = a->rht_signs;
+  if (P.segm_rows > 0) {  // no more segments than keep the device's CUs busy, as the workspace grows with them
+    const int64_t pairs = (int64_t)a->num_seqs * cache->num_kv_heads;
+    const int64_t want = (8 * (int64_t)device_cus() + pairs - 1) / pairs;
+    if (want < d.num_segments) d.num_segments = (int)want;
+  }
 
   qp_prefill_args &f = P.prefill;
   f.query = a->query;
@@ -134,11 +189,13 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
   f.rht_out_scale = a->rht_out_scale;
   f.query_signs = a->rht_signs;
 
-  // workspace: [route_row | row_tok | row_seq | prefill workspace]
+  // workspace: [route_row | row_tok | row_seq | split-KV partials | prefill workspace]
   P.off_route = 0;
   P.off_tok = P.routed ? up256(4 * (int64_t)a->num_seqs) : 0;
   P.off_seq = P.off_tok + (P.routed ? up256(4 * (int64_t)P.rows_cap) : 0);
-  P.off_prefill = P.off_seq + (P.routed ? up256(4 * (int64_t)P.rows_cap) : 0);
+  P.off_segm = P.off_seq + (P.routed ? up256(4 * (int64_t)P.rows_cap) : 0);
+  P.off_prefill =
+      P.off_segm + (P.segm_rows > 0 ? segm_bytes(P.segm_rows * a->num_q_heads * P.decode.num_segments, hs) : 0);
   const int64_t pf = P.plain_decode ? 0 : qp_prefill_workspace_size(cache, &f);
   P.total = pf > 0 ? P.off_prefill + up256(pf) : P.off_prefill;
   f.workspace_bytes = pf;
@@ -165,6 +222,7 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
   if (P.total > 0)
     QP_REQUIRE(ws && a->workspace_bytes >= P.total && aligned(ws, 256),
                "qp_attention: this batch needs a 256-byte aligned workspace of qp_attention_workspace_size bytes");
+  if (P.segm_rows > 0) segm_in_workspace(P, cache, ws);
   const int G = a->num_q_heads / cache->num_kv_heads;
   const int max_rows = a->max_decode_rows > 0 && a->max_decode_rows < 32 ? a->max_decode_rows : 32;
   if (P.plain_decode) {
@@ -173,25 +231,7 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
     const bool groups = rows > max_rows || (rows > 16 && cache->head_size == 512);
     int st = groups ? decode_routed(cache, &P.decode, nullptr, max_rows, s) : qp_decode_splitkv(cache, &P.decode, stream);
     if (st != QP_OK) return st;
-    qp_merge_args m = {};
-    m.segm_output = a->segm_output;
-    for (int i = 0; i < 3; ++i) m.segm_output_stride[i] = a->segm_output_stride[i];
-    m.segm_max = a->segm_max;
-    m.segm_expsum = a->segm_expsum;
-    m.segm_stat_stride[0] = a->segm_stat_stride[0];
-    m.segm_stat_stride[1] = a->segm_stat_stride[1];
-    m.cu_seqlens_q = a->cu_seqlens_q;
-    m.seqused_k = a->seqused_k;
-    m.num_seqs = a->num_seqs;
-    m.num_tokens = a->num_tokens;
-    m.num_q_heads = a->num_q_heads;
-    m.head_size = cache->head_size;
-    m.num_segments = a->num_segments;
-    m.out = a->out;
-    m.out_stride[0] = a->out_stride[0];
-    m.out_stride[1] = a->out_stride[1];
-    m.rht_signs = a->rht_signs;
-    m.rht_out_scale = a->rht_out_scale;
+    const qp_merge_args m = merge_of(P.decode, a, cache->head_size);
     return qp_merge_segments(&m, stream);
   }
   P.prefill.workspace = P.prefill.workspace_bytes > 0 ? ws + P.off_prefill : nullptr;
@@ -209,25 +249,7 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
   // each short sequence's query count here
   st = decode_routed(cache, &P.decode, route_row, 16, s);
   if (st != QP_OK) return st;
-  qp_merge_args m = {};
-  m.segm_output = a->segm_output;
-  for (int i = 0; i < 3; ++i) m.segm_output_stride[i] = a->segm_output_stride[i];
-  m.segm_max = a->segm_max;
-  m.segm_expsum = a->segm_expsum;
-  m.segm_stat_stride[0] = a->segm_stat_stride[0];
-  m.segm_stat_stride[1] = a->segm_stat_stride[1];
-  m.cu_seqlens_q = a->cu_seqlens_q;
-  m.seqused_k = a->seqused_k;
-  m.num_seqs = a->num_seqs;
-  m.num_tokens = a->num_tokens;
-  m.num_q_heads = a->num_q_heads;
-  m.head_size = cache->head_size;
-  m.num_segments = a->num_segments;
-  m.out = a->out;
-  m.out_stride[0] = a->out_stride[0];
-  m.out_stride[1] = a->out_stride[1];
-  m.rht_signs = a->rht_signs;
-  m.rht_out_scale = a->rht_out_scale;
+  const qp_merge_args m = merge_of(P.decode, a, cache->head_size);
   return merge_routed(&m, row_tok, row_seq, P.rows_cap, nullptr, s);
 }
 

@@ -13,8 +13,8 @@ This package replaces the whole read path with hand-written gfx950 kernels reach
 
 The arithmetic is the reference's exact kernel: bf16 query and exact-integer nibble operands, fp32 accumulation, and
 the value zero point removed with the same bf16-rounded P * s_v that feeds the PV product (int4_kv.py:80-95).
-Nothing here copies to or waits for the host; a batch of short sequences allocates nothing either, so decode steps
-can be captured in HIP graphs.
+Nothing here copies to or waits for the host; a batch of short sequences that fits the segment buffers allocates
+nothing either, so decode steps can be captured in HIP graphs.
 """
 from __future__ import annotations
 
@@ -173,7 +173,7 @@ def _scratch():
 def attend(q, k_cache, v_cache, k_scale_cache, v_scale_cache, out, **kw) -> None:
     """One qp_attention call (see attention_args for the keywords): the library routes the batch between split-KV
     decode and prefill on the device. A workspace is taken from torch's caching allocator only when the batch has
-    sequences of more than 4 query tokens (a batch of short sequences needs none)."""
+    sequences of more than 4 query tokens, or more rows of short sequences than the segment buffers hold."""
     cache, args = _scratch()
     _hip.pack_paged_cache(cache, k_cache, v_cache, k_scale_cache, v_scale_cache, q.shape[2])
     _pack_attention(args, q, out, **kw)
@@ -227,7 +227,8 @@ def unified_attention_int4(q, k_cache, v_cache, out, *, cu_seqlens_q, max_seqlen
     One library call: sequences with at most MAX_Q_SPLIT_KV query tokens take the split-KV decode (when the caller
     passes segment buffers; int4_kv.py:101-112 and the sub-batch of :308-323), the others the MFMA prefill kernel,
     both routed on the device. q is rotated as the kernels load it and the output rotated back before its store
-    (single_rht framing, :326-329). No host synchronisation; no allocation for a batch of short sequences."""
+    (single_rht framing, :326-329). No host synchronisation; no allocation for a batch of short sequences whose rows
+    fit the segment buffers (a larger one takes its partials' workspace from torch's caching allocator)."""
     del use_alibi_sqrt, seq_threshold_3D, kw
     _plain(q, window_size, softcap, sinks, alibi_slopes, qq_bias, output_scale, mm_prefix_range)
     _check_batch(q, cu_seqlens_q, seqused_k, block_table)
