@@ -43,6 +43,38 @@ constexpr float kPfRescale = 64.f;  // log2 headroom before the running maximum 
 // exist in the sequence's block-table row.
 constexpr int kPfSteadyLead = 7;
 
+// row_pos of a row past the block's last (token, head) pair: below every key, as a row without keys, but not stored
+constexpr int kPfNoRow = -0x7FFFFFFF - 1;
+
+// The per-key scalars of the softmax, from the key's and value's scale words:
+//   a = s_k scale log2(e) and e = a (128 + zp_k) (int8 keys: 128 a), so that the score is raw a - qsum e;
+//   b = log2(s_v) / a, the start value of the key's QK accumulator: the score then carries log2(s_v), and one exp2
+//     gives P s_v, the value probability, without a multiply;
+//   r = 1 / s_v as two bf16 halves (hi + lo, 16 bits), two rows of the zero-point tile: the PV MFMA then sums
+//     P16 / s_v, the row's l, without a VALU add per key.
+// A key past the split's end gets zeros. The store floors both scales at 1e-6, so a written key has a, s_v > 0; a
+// zero scale (never written) yields b = 0 and r = 0 rather than an infinity. b and r use v_rcp_f32 (about 1 ulp):
+// b's error then moves the score by about |log2 s_v| 2^-23 log2 units, and r is kept to 16 bits anyway.
+template <int KFMT>
+__device__ __forceinline__ void pf_key_scalars(uint32_t kw, uint32_t vw, float scale_log2, bool ok, float &a, float &e,
+                                               float &b, uint16_t &rhi, uint16_t &rlo) {
+  if constexpr (KFMT == QP_CODES_INT4) {
+    a = __uint_as_float(kw & 0xFFFFFFF0u) * scale_log2;
+    e = a * (float)(128u + (kw & 0xFu));
+  } else {
+    a = __uint_as_float(kw) * scale_log2;
+    e = a * 128.f;  // the operands are 128 + k
+  }
+  const float sv = __uint_as_float(vw & 0xFFFFFFF0u);
+  const bool fine = ok && sv > 0.f && a > 1e-30f;
+  b = fine ? __builtin_amdgcn_logf(sv) * __builtin_amdgcn_rcpf(a) : 0.f;
+  const float r = fine ? __builtin_amdgcn_rcpf(sv) : 0.f;
+  rhi = f32_to_bf16_bits(r);
+  rlo = f32_to_bf16_bits(r - __uint_as_float((uint32_t)rhi << 16));
+  a = ok ? a : 0.f;
+  e = ok ? e : 0.f;
+}
+
 template <int HS, int KFMT>
 struct PfShape {
   static constexpr int kHS = HS;
@@ -177,11 +209,11 @@ __device__ __forceinline__ void pf_slots(const PrefillParams &p, int k0, int ken
 }
 
 // Strided fallback: the same packed image gathered dword by dword through VGPRs (any 4-byte aligned views).
-template <class Sh>
+template <class Sh, int KEYS = kPfKeys, int THREADS = kPfWaves * 64>
 __device__ __forceinline__ void pf_gather(const PrefillParams &p, const int32_t *trow, int k0, int kend, int h,
                                           uint8_t *pk) {
   constexpr int kDw = Sh::kCell / 4, kKd = Sh::kKeyBytes / 4, kVd = Sh::kHS / 8;
-  for (int u = threadIdx.x; u < kPfKeys * kDw; u += kPfWaves * 64) {
+  for (int u = threadIdx.x; u < KEYS * kDw; u += THREADS) {
     const int kk = u / kDw, d = u % kDw;
     const int key = min(k0 + kk, kend - 1);
     const int bidx = fast_div(key, p.bs_magic, p.bs_shift);
@@ -219,9 +251,14 @@ PrefillParams prefill_params(const qp_paged_cache *cache, const qp_prefill_args 
 // The log-sum-exp merge of a split prefill's partials into a->out (inverse rotation when a->rht_signs is set).
 int prefill_merge(const PrefillParams &p, const qp_prefill_args *a, int hs, const int32_t *skip_seq, hipStream_t s);
 
-// The prefill on 32x32x16 MFMAs (qp_prefill_wide.hip), head 128, or 512 with int4 keys (at least 2 key splits): grid
-// (row blocks of prefill_wide_rows(head size) (token, query head) pairs, KV heads, key splits).
-int prefill_wide_rows(int head_size);
-void prefill_wide(const PrefillParams &p, int head_size, int key_format, dim3 grid, bool span, hipStream_t s);
+// The prefill on 32x32x16 MFMAs (qp_prefill_wide.hip), head 512 with int4 keys (at least 2 key splits): grid (row blocks
+// of prefill_wide_rows() (token, query head) pairs, KV heads, key splits).
+int prefill_wide_rows();
+void prefill_wide(const PrefillParams &p, dim3 grid, bool span, hipStream_t s);
+
+// The prefill with two waves per SIMD (qp_prefill_dual.hip), heads 64 and 128: grid (row blocks of prefill_dual_rows()
+// (token, query head) pairs, KV heads, key splits).
+int prefill_dual_rows();
+void prefill_dual(const PrefillParams &p, int head_size, int key_format, dim3 grid, bool span, hipStream_t s);
 
 }  // namespace qp

@@ -46,38 +46,6 @@
 
 namespace qp {
 
-// row_pos of a row past the block's last (token, head) pair: below every key, as a row without keys, but not stored
-constexpr int kPfNoRow = -0x7FFFFFFF - 1;
-
-// The per-key scalars of the softmax, from the key's and value's scale words:
-//   a = s_k scale log2(e) and e = a (128 + zp_k) (int8 keys: 128 a), so that the score is raw a - qsum e;
-//   b = log2(s_v) / a, the start value of the key's QK accumulator: the score then carries log2(s_v), and one exp2
-//     gives P s_v, the value probability, without a multiply;
-//   r = 1 / s_v as two bf16 halves (hi + lo, 16 bits), two rows of the zero-point tile: the PV MFMA then sums
-//     P16 / s_v, the row's l, without a VALU add per key.
-// A key past the split's end gets zeros. The store floors both scales at 1e-6, so a written key has a, s_v > 0; a
-// zero scale (never written) yields b = 0 and r = 0 rather than an infinity. b and r use v_rcp_f32 (about 1 ulp):
-// b's error then moves the score by about |log2 s_v| 2^-23 log2 units, and r is kept to 16 bits anyway.
-template <int KFMT>
-__device__ __forceinline__ void pf_key_scalars(uint32_t kw, uint32_t vw, float scale_log2, bool ok, float &a, float &e,
-                                               float &b, uint16_t &rhi, uint16_t &rlo) {
-  if constexpr (KFMT == QP_CODES_INT4) {
-    a = __uint_as_float(kw & 0xFFFFFFF0u) * scale_log2;
-    e = a * (float)(128u + (kw & 0xFu));
-  } else {
-    a = __uint_as_float(kw) * scale_log2;
-    e = a * 128.f;  // the operands are 128 + k
-  }
-  const float sv = __uint_as_float(vw & 0xFFFFFFF0u);
-  const bool fine = ok && sv > 0.f && a > 1e-30f;
-  b = fine ? __builtin_amdgcn_logf(sv) * __builtin_amdgcn_rcpf(a) : 0.f;
-  const float r = fine ? __builtin_amdgcn_rcpf(sv) : 0.f;
-  rhi = f32_to_bf16_bits(r);
-  rlo = f32_to_bf16_bits(r - __uint_as_float((uint32_t)rhi << 16));
-  a = ok ? a : 0.f;
-  e = ok ? e : 0.f;
-}
-
 // K part of the unpack: bf16 K rows kd[key][channel], 8 channels per dword of int4 codes (4 of int8).
 template <int HS, int KFMT>
 __device__ __forceinline__ void pf_unpack_k(const uint8_t *pk, uint8_t *kd, int tid) {
@@ -254,8 +222,7 @@ struct PfStager {
 // destination within 18 wait states and fails if it finds one.
 template <int NT>
 __device__ __forceinline__ void pv_step(f32x4_t (&acc)[NT][17], int b, bf16x8_t vop, const u32x4_t (&pop)[NT]) {
-  static_assert(NT >= 1 && NT <= 4, "row tiles");
-  // (the accumulator array is sized for head 256; head 128 uses tiles 0..8)
+  static_assert(NT >= 1 && NT <= 3, "row tiles");
   // One statement per MFMA, so that VALU work can be placed between them.
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -280,8 +247,7 @@ template <int NT>
 __device__ __forceinline__ void p_ready(u32x4_t (&pop)[NT]) {
   if constexpr (NT == 1) asm volatile("s_nop 1" : "+v"(pop[0]));
   else if constexpr (NT == 2) asm volatile("s_nop 1" : "+v"(pop[0]), "+v"(pop[1]));
-  else if constexpr (NT == 3) asm volatile("s_nop 1" : "+v"(pop[0]), "+v"(pop[1]), "+v"(pop[2]));
-  else asm volatile("s_nop 1" : "+v"(pop[0]), "+v"(pop[1]), "+v"(pop[2]), "+v"(pop[3]));
+  else asm volatile("s_nop 1" : "+v"(pop[0]), "+v"(pop[1]), "+v"(pop[2]));
 }
 
 // one QK step (32 channels of one 16-key sub-tile) for every row tile of the wave
@@ -890,26 +856,23 @@ using namespace qp;
 
 namespace {
 
-// Row tiles per wave: 3 (192 (token, query head) rows per workgroup), or fewer when the longest chunk holds fewer rows.
-// At head 128 a chunk of more than 192 rows takes 4 (256 rows; 148 AGPRs and 256 VGPRs, no spill): 2.86-2.89 against
-// 3.00-3.04 ms on a 1024-token chunk of 32 q / 8 KV heads over 131072 keys, with the splits below.
-int prefill_nt(int G, int max_query_len, int hs) {
+// Row tiles per wave of the tile kernel: 3 (192 (token, query head) rows per workgroup), or fewer when the longest chunk
+// holds fewer rows.
+int prefill_nt(int G, int max_query_len) {
   const int64_t rows = (int64_t)(max_query_len > 0 ? max_query_len : 1) * G;
-  if (hs == 128 && rows > 192) return 4;
   return rows > 128 ? 3 : rows > 64 ? 2 : 1;
 }
 
-// Key splits per row block of the tile kernel.
+int64_t rows_per_block(int hs, int nt) {
+  return hs == 512 ? prefill_wide_rows() : hs == 256 ? (int64_t)kPfWaves * 16 * nt : prefill_dual_rows();
+}
+
+// Key splits per row block of the tile and dual kernels.
 int prefill_splits(const qp_paged_cache *cache, const qp_prefill_args *a, int nt) {
   if (a->num_splits > 0) return a->num_splits;
-  const int64_t rows = (int64_t)kPfWaves * 16 * nt;
+  const int64_t rows = rows_per_block(cache->head_size, nt);
   const int64_t blocks = ((int64_t)a->num_tokens * (a->num_q_heads / cache->num_kv_heads) + rows - 1) / rows;
-  // four row tiles: splits of at most about 300 tiles (9600 keys). With the 2 splits the rounds alone give, each
-  // workgroup streamed 2064 tiles, 8.9 MB of keys and values that its row-block neighbours no longer shared through
-  // L2, and the chunk above took 4.81 ms; 8 splits 3.06 ms, 14 splits 2.87 ms. (Three row tiles gain nothing from
-  // more splits.)
-  const int min_s = nt == 4 ? (int)std::min<int64_t>(64, std::max<int64_t>(1, ((int64_t)a->max_seqlen_k + 9599) / 9600)) : 1;
-  return balanced_splits(blocks * cache->num_kv_heads, a, min_s);
+  return balanced_splits(blocks * cache->num_kv_heads, a, 1);
 }
 
 int64_t partial_bytes(const qp_paged_cache *cache, const qp_prefill_args *a, int splits) {
@@ -929,41 +892,38 @@ template <int HS, int KFMT>
 void dispatch_nt(const PrefillParams &p, int nt, dim3 grid, bool span, hipStream_t s) {
   if (nt == 1) launch_prefill<HS, KFMT, 1>(p, grid, span, s);
   else if (nt == 2) launch_prefill<HS, KFMT, 2>(p, grid, span, s);
-  else if constexpr (HS == 128) {
-    if (nt == 4) launch_prefill<HS, KFMT, 4>(p, grid, span, s);
-    else launch_prefill<HS, KFMT, 3>(p, grid, span, s);
-  } else {
-    launch_prefill<HS, KFMT, 3>(p, grid, span, s);
-  }
+  else launch_prefill<HS, KFMT, 3>(p, grid, span, s);
 }
 
-// Which kernel serves a prefill (measured over 1024-token chunks at contexts of 32768 and 131072 keys):
-//   * head 256, and head 128 below 8 query heads per KV head: the 16-row-tile kernel above, whose 192-row blocks hold
-//     (token, head) pairs at any GQA width. At head 256 with 16 heads per KV head it takes 1.63 ms against the wide
-//     kernel's 1.72 (one 32-row tile per wave there: each K / V operand read from LDS serves 32 rows against 48);
-//   * head 128 from 8 query heads per KV head, and head 512 with int4 keys: the wide kernel (qp_prefill_wide.hip,
-//     32x32x16 MFMAs, 64 rows per wave at head 128): 1.77 against 1.97 ms at 8 heads per KV head, 0.94 against 1.29
-//     at 16;
-//   * head 512 with int8 keys, whose 776-byte cells do not fit the wide kernel's LDS plan, and head 64, whose 4 QK
-//     steps per tile leave the MFMA kernels' unpack nothing to hide behind: query slices of the split-KV kernel.
-enum class PrefillPath { kSlices, kTiles, kWide };
+// Which kernel serves a prefill:
+//   * heads 64 and 128: the dual kernel (qp_prefill_dual.hip), two waves per SIMD, at every GQA width and chunk length.
+//     2048 tokens over 16384 keys with 64 q / 8 KV heads of 128: 1.22-1.31 ms against 1.96 on the wide kernel's 32x32x16
+//     MFMAs with one wave per SIMD; 8 prompts of up to 2048 tokens with 32 q / 8 KV heads: 147 against 265 us on four
+//     16-row tiles per wave of the tile kernel; 512 tokens over 4096 keys with 32 q / 8 KV heads of 64: 58 against 94 us
+//     as query slices;
+//   * head 256, whose accumulators and query operands leave room for one wave per SIMD: the tile kernel above, whose
+//     192-row blocks hold (token, head) pairs at any GQA width. With 16 heads per KV head it takes 1.63 ms against
+//     1.72 on 32x32x16 MFMAs (one 32-row tile per wave there: each K / V operand read from LDS serves 32 rows against
+//     48);
+//   * head 512 with int4 keys: the wide kernel (qp_prefill_wide.hip, 32x32x16 MFMAs);
+//   * head 512 with int8 keys, whose 776-byte cells do not fit the wide kernel's LDS plan: query slices of the
+//     split-KV kernel.
+enum class PrefillPath { kSlices, kTiles, kWide, kDual };
 
 PrefillPath prefill_path(const qp_paged_cache *cache, const qp_prefill_args *a) {
   const int hs = cache->head_size;
   if (hs == 512) return cache->key.format == QP_CODES_INT4 ? PrefillPath::kWide : PrefillPath::kSlices;
-  if (hs == 128) return a->num_q_heads / cache->num_kv_heads >= 8 ? PrefillPath::kWide : PrefillPath::kTiles;
-  return hs == 256 ? PrefillPath::kTiles : PrefillPath::kSlices;
+  return hs == 256 ? PrefillPath::kTiles : PrefillPath::kDual;
 }
 
-// Key splits of the wide kernel, as balanced_splits (192 workgroups on 256 CUs: 4 splits, 3 full rounds). At head 512
-// at least 2: that kernel writes split partials only, and the merge rotates and normalises.
+// Key splits of the wide kernel, as balanced_splits (192 workgroups on 256 CUs: 4 splits, 3 full rounds), at least 2: it
+// writes split partials only, and the merge rotates and normalises.
 int wide_splits(const qp_paged_cache *cache, const qp_prefill_args *a) {
-  const int min_s = cache->head_size == 512 ? 2 : 1;
-  if (a->num_splits > 0) return a->num_splits > min_s ? a->num_splits : min_s;
+  if (a->num_splits > 0) return a->num_splits > 2 ? a->num_splits : 2;
   const int G = a->num_q_heads / cache->num_kv_heads;
-  const int rows = prefill_wide_rows(cache->head_size);
+  const int rows = prefill_wide_rows();
   const int64_t blocks = ((int64_t)a->num_tokens * G + rows - 1) / rows;
-  return balanced_splits(blocks * cache->num_kv_heads, a, min_s);
+  return balanced_splits(blocks * cache->num_kv_heads, a, 2);
 }
 
 }  // namespace
@@ -975,7 +935,7 @@ extern "C" int64_t qp_prefill_workspace_size(const qp_paged_cache *cache, const 
   if (path == PrefillPath::kSlices) return slice_prefill_workspace(cache, a);
   if (path == PrefillPath::kWide) return partial_bytes(cache, a, wide_splits(cache, a));
   return partial_bytes(cache, a, prefill_splits(cache, a, prefill_nt(a->num_q_heads / cache->num_kv_heads,
-                                                                    a->max_query_len, cache->head_size)));
+                                                                    a->max_query_len)));
 }
 
 namespace qp {
@@ -1092,13 +1052,13 @@ int prefill_run(const qp_paged_cache *cache, const qp_prefill_args *a, const int
   const PrefillPath path = prefill_path(cache, a);
   if (path == PrefillPath::kSlices) return slice_prefill(cache, a, skip_seq, s);
   const bool wide = path == PrefillPath::kWide;
-  const int nt = wide ? 0 : prefill_nt(G, a->max_query_len, hs);
+  const int nt = prefill_nt(G, a->max_query_len);
   int splits = wide ? wide_splits(cache, a) : prefill_splits(cache, a, nt);
   if (splits > 1 && (!a->workspace || a->workspace_bytes < partial_bytes(cache, a, splits))) {
     QP_REQUIRE(a->num_splits == 0, "qp_prefill: workspace too small for the requested splits");
     splits = 1;  // automatic choice without (enough) workspace: one workgroup per query block and KV head
   }
-  QP_REQUIRE(!wide || hs != 512 || splits > 1,
+  QP_REQUIRE(!wide || splits > 1,
              "qp_prefill: head 512 needs a workspace of qp_prefill_workspace_size bytes (split partials)");
   QP_REQUIRE(splits == 1 || aligned(a->workspace, 16), "qp_prefill: workspace must be 16-byte aligned");
 
@@ -1106,18 +1066,17 @@ int prefill_run(const qp_paged_cache *cache, const qp_prefill_args *a, const int
   p.skip_seq = skip_seq;
   // sequence s owns row blocks [cu_q[s] G / R + s, cu_q[s + 1] G / R + s + 1) of R rows each: an upper bound known on
   // the host
-  const int64_t rows_per_block = wide ? prefill_wide_rows(hs) : (int64_t)kPfWaves * 16 * nt;
-  const unsigned blocks = (unsigned)((int64_t)a->num_tokens * G / rows_per_block + a->num_seqs);
+  const unsigned blocks = (unsigned)((int64_t)a->num_tokens * G / rows_per_block(hs, nt) + a->num_seqs);
   const dim3 grid(blocks, cache->num_kv_heads, splits);
   const bool span = is_span_layout(cache) && cache->key.code_stride[0] < (int64_t(1) << 31);
   if (wide) {
-    prefill_wide(p, hs, cache->key.format, grid, span, s);
-  } else if (hs == 256) {
-    if (cache->key.format == QP_CODES_INT4) dispatch_nt<256, QP_CODES_INT4>(p, nt, grid, span, s);
-    else dispatch_nt<256, QP_CODES_INT8>(p, nt, grid, span, s);
+    prefill_wide(p, grid, span, s);
+  } else if (path == PrefillPath::kDual) {
+    prefill_dual(p, hs, cache->key.format, grid, span, s);
+  } else if (cache->key.format == QP_CODES_INT4) {
+    dispatch_nt<256, QP_CODES_INT4>(p, nt, grid, span, s);
   } else {
-    if (cache->key.format == QP_CODES_INT4) dispatch_nt<128, QP_CODES_INT4>(p, nt, grid, span, s);
-    else dispatch_nt<128, QP_CODES_INT8>(p, nt, grid, span, s);
+    dispatch_nt<256, QP_CODES_INT8>(p, nt, grid, span, s);
   }
   const int st = launch_status();
   if (st != QP_OK) return st;

@@ -1,44 +1,37 @@
-// Chunked-prefill attention over the paged int4 / k8v4 KV cache on 32x32x16 bf16 MFMAs, 64 query rows per wave.
+// Chunked-prefill attention over the paged int4 KV cache at head 512, on 32x32x16 bf16 MFMAs, 32 query rows per wave.
 //
 // Reference semantics: as prefill_kernel (qp_prefill.hip): the exact kernel's arithmetic (int4_kv.py:80-95,127-142)
 // for long chunks, replacing the reference's unpack-then-FlashAttention detour (int4_prefill.py:203-232): bf16 query
-// and exact-integer code operands, fp32 accumulation, S = (q . (128 + k) - sum(q) (128 + zp_k)) s_k scale (int4 keys)
-// or (q . (128 + k) - 128 sum(q)) s_k scale (int8 keys), P_v16 = bf16(P s_v) feeding both the PV product and the
-// zero-point sum (int4_kv.py:90-94), l from the unrounded P, causal within each sequence's query chunk.
+// and exact-integer code operands, fp32 accumulation, S = (q . (128 + k) - sum(q) (128 + zp_k)) s_k scale, P_v16 =
+// bf16(P s_v) feeding both the PV product and the zero-point sum (int4_kv.py:90-94), l from the unrounded P, causal
+// within each sequence's query chunk.
 //
-// MI355X design (heads 128 and 512; head 256 runs on the 16-row-tile kernel, which serves it faster at every GQA
-// width). A workgroup of 4 waves (one per SIMD) owns 128 NT query rows of one KV head and one key split; the rows are
-// the chunk's (token, query head) pairs in token-major order, so any GQA group width packs them densely. Wave w holds
-// NT 32-row tiles (NT = 2 at head 128: 32 VGPRs of query operands and 64 AGPRs of accumulators per tile; NT = 1 at
-// head 512, below):
-//   * S^T = K Q^T on v_mfma_f32_32x32x16_bf16: the K tile (32 keys x 16 channels) is the A operand, read from LDS
-//     once per step and used by every row tile; the query rows are the B operand, held in VGPRs; these MFMAs are
-//     inline assembly writing VGPRs, so the compiler's own MFMAs (the PV below) keep AGPR accumulators;
+// MI355X design. A workgroup of 4 waves (one per SIMD) owns 128 query rows of one KV head and one key split; the rows are
+// the chunk's (token, query head) pairs in token-major order, so any GQA group width packs them densely. A wave holds one
+// 32-row tile: 128 VGPRs of query operands and all 256 AGPRs of accumulators.
+//   * S^T = K Q^T on v_mfma_f32_32x32x16_bf16: the K tile (32 keys x 16 channels) is the A operand; the query rows are the
+//     B operand, held in VGPRs; these MFMAs are inline assembly writing VGPRs, so that the PV accumulators keep the AGPRs;
 //   * the S^T accumulator (lane l: row l % 32, keys 8 (i / 4) + 4 (l / 32) + i % 4) is, packed to bf16 P16, exactly
 //     the B operand of O^T += V^T P^T for the 16 keys of each K step, so P never leaves registers; the V^T rows in
 //     LDS hold their 32 keys in that order;
-//   * the O^T accumulators (NT x HS / 32 channel tiles of 16 AGPRs) are the compiler's; nothing in the loop reads them
-//     from C++, so they stay in place;
+//   * nothing in the loop reads the O^T accumulators (16 channel tiles of 16 AGPRs) from C++, so they stay in place;
 //   * the zero-point sum sum_k P16_k (16 + zp_v,k) is a v_dot2 of the same P16 pairs against (16 + zp) pairs.
 // Measured on one wave per SIMD, a 32x32x16 MFMA runs at the full 32 cycles back to back and hides about four
 // independent VALU instructions and most of an exp2, where eight 16x16x32 MFMAs of the same FLOPs take 152 cycles
-// and an interleaved exp2 costs about 11 cycles; with 64 rows per wave each K / V operand read and each unpacked
-// tile serve a third more rows than with 48.
+// and an interleaved exp2 costs about 11 cycles.
 // Per 32-key tile, one barrier: the tile's page runs come HBM -> LDS four tiles ahead (the copy plan and block-table
-// walk of PfCopies / kPfSteadyLead), all 256 threads unpack tile i + 2 to exact bf16 integers (K rows 128 + n, V^T rows
-// 16 + n, per-key scalars) while the waves run S^T of tile i + 1, then O^T += V^T P^T of tile i runs beside the softmax
-// of tile i + 1.
-// Head 512 (int4 keys; one 32-row tile per wave: 128 VGPRs of query operands, all 256 AGPRs of accumulators): two bf16
-// K buffers would not fit beside the V^T buffers in the 160 KB, so each wave builds its K operands from the packed codes
-// in LDS (one 8-byte read per two steps, four v_bitop3 per step, as the unpack would), V^T is unpacked one tile ahead
-// into two buffers and the per-key scalars two tiles ahead into a ring of two: 4 packed slots + 2 V^T buffers + the
-// ring = 146 KB. That kernel always runs key-split: the merge normalises and rotates its 512-channel rows.
+// walk of PfCopies / kPfSteadyLead), S^T of tile i + 1 runs beside the unpack, then O^T += V^T P^T of tile i beside the
+// softmax of tile i + 1. Two bf16 K buffers would not fit beside the V^T buffers in the 160 KB, so each wave builds its K
+// operands from the packed codes in LDS (one 8-byte read per two steps, four v_bitop3 per step, as an unpack would), V^T
+// is unpacked one tile ahead into two buffers (V^T rows 16 + n) and the per-key scalars two tiles ahead into a ring of
+// two: 4 packed slots + 2 V^T buffers + the ring = 146 KB. The kernel always runs key-split: the merge normalises and
+// rotates its 512-channel rows.
 // The running maximum m of a row starts kWideBias log2 units above the first tile's maximum, and probabilities are
 // taken as 2^(s - m) as long as no score exceeds m by more than kWideHeadroom (fp32 then holds l, the zero-point sum and
-// the accumulators over 2^17 keys: below 2^122). A score beyond (136 units above the first tile's maximum; never seen
-// on the synthetic k8v4 caches, whose scores reach about 100) sets a workgroup word: after the next barrier every
-// wave starts the split again with its rows' maxima raised, and the accumulators are only zeroed, never rescaled in
-// the loop (a rescale there, C++ access to the AGPR tiles, made the register allocator spill them).
+// the accumulators over 2^17 keys: below 2^122). A score beyond (136 units above the first tile's maximum) sets a
+// workgroup word: after the next barrier every wave starts the split again with its rows' maxima raised, and the
+// accumulators are only zeroed, never rescaled in the loop (a rescale there, C++ access to the AGPR tiles, made the
+// register allocator spill them).
 #include "qp_prefill.h"
 
 #include <type_traits>
@@ -52,75 +45,49 @@ constexpr int kWidePasses = 8;         // passes over a split at most (each rais
 template <int HS, int KFMT>
 struct WShape {
   using Pf = PfShape<HS, KFMT>;
-  // Head 512 (int4 keys): bf16 K rows do not fit beside the V^T buffers, so each wave builds its QK operands from the
-  // packed codes (K direct), V is unpacked one tile ahead into two buffers and the per-key scalars two tiles ahead into
-  // a ring of two, and the packed slots (4) hold the tiles from the one being read to the one being copied.
-  static constexpr bool kDirect = HS == 512;
-  static_assert(!kDirect || KFMT == QP_CODES_INT4, "head 512 takes int4 keys");
+  static_assert(HS == 512 && KFMT == QP_CODES_INT4, "head 512 with int4 keys");
   static constexpr int kKeyBytes = Pf::kKeyBytes;
   static constexpr int kCell = Pf::kCell;
-  static constexpr int kSlot = kDirect ? 32 * kCell : Pf::kPk;  // one packed slot (two 16-cell page runs)
-  static constexpr int kSlots = kDirect ? 4 : 3;
-  static constexpr int kKdRow = HS * 2 + 16;       // bf16 K row + 16 bytes: 32 rows at one column hit 32 bank quads
-  static constexpr int kKd = kPfKeys * kKdRow;
+  static constexpr int kSlot = 32 * kCell;         // one packed slot (two 16-cell page runs)
+  // the packed slots hold the tiles from the one being read to the one being copied
+  static constexpr int kSlots = 4;
   static constexpr int kVtRow = kPfKeys * 2 + 16;  // 80 B: 32 rows x 16 B reads at one column are conflict-free
   static constexpr int kVt = HS * kVtRow;
   // per-key scalars of a tile: a_k, e_k, s_v (fp32 [32] each), then bf16 16 + zp_v in lane order [32], then a dummy
-  // slot for the threads that own no key; after the V^T rows of the tile's V buffer, or in the ring (K direct)
+  // slot for the threads that own no key; in the ring
   static constexpr int kScA = 0, kScE = 128, kScS = 256, kScZ = 384, kScDummy = 448, kSc = 512;
-  static constexpr int kVb = kDirect ? kVt : kVt + kSc;
-  static constexpr int kVbufs = kDirect ? 2 : 3;
-  static constexpr int kOffK = kSlots * kSlot;      // packed slots, 2 K buffers (not K direct), V buffers, the ring
-  static constexpr int kOffV = kOffK + (kDirect ? 0 : 2 * kKd);
+  static constexpr int kVb = kVt;
+  static constexpr int kVbufs = 2;
+  static constexpr int kOffV = kSlots * kSlot;      // packed slots, V buffers, the ring
   static constexpr int kOffR = kOffV + kVbufs * kVb;
-  static constexpr int kLds = kOffR + (kDirect ? 2 * kSc : 0);
-  static_assert(kSlot % 16 == 0 && kKd % 16 == 0 && kVb % 16 == 0, "alignment");
+  static constexpr int kLds = kOffR + 2 * kSc;
+  static_assert(kSlot % 16 == 0 && kVb % 16 == 0, "alignment");
   static_assert(kLds <= 160 * 1024, "LDS");
   // key of PV slot s (0..15) of K step ks for lane half h: the S^T row order of the 32x32 accumulator
   static constexpr __host__ __device__ int slot_key(int ks, int h, int s) { return 16 * ks + (s < 4 ? 4 * h + s : 4 + 4 * h + s); }
-  // first channel (in K operand order) of QK step cs for lane half h: consecutive code dwords of a key go to the
-  // lane's consecutive steps when the operands come from the packed codes, so one 8-byte read serves two steps
-  static constexpr __host__ __device__ int step_chan(int cs, int h) { return kDirect ? 8 * (HS / 16 * h + cs) : 16 * cs + 8 * h; }
+  // first channel (in K operand order) of QK step cs for lane half h: consecutive code dwords of a key go to the lane's
+  // consecutive steps, so one 8-byte read serves two steps
+  static constexpr __host__ __device__ int step_chan(int cs, int h) { return 8 * (HS / 16 * h + cs); }
 };
 
 // Position of key kk's 16 + zp_v in the lane-ordered zero-point row: lane half h reads its 16 keys' values as i = 0..15
 // (key 8 (i / 4) + 4 h + i % 4) from 32 bytes at 32 h.
 __host__ __device__ constexpr int zp_pos(int kk) { return 16 * ((kk >> 2) & 1) + 4 * (kk >> 3) + (kk & 3); }
 
-// The unpack of one tile, cut into stages that the QK phase spreads over its MFMA steps. The per-key scalars come from
-// slot pks into block sc (the same tile as the codes, or two tiles ahead of V with K direct).
+// The unpack of one tile's V, cut into stages that the QK phase spreads over its MFMA steps. The per-key scalars come from
+// slot pks into block sc (a tile further on).
 template <int HS, int KFMT>
 struct WStager {
   using Sh = WShape<HS, KFMT>;
-  static constexpr int kKDw = KFMT == QP_CODES_INT4 ? HS / 8 : HS / 4;  // code dwords per key
-  static constexpr int kNK = kPfKeys * kKDw / (kPfWaves * 64);           // K dwords per thread
   static constexpr int kVUnits = HS > kPfWaves * 64 ? HS / (kPfWaves * 64) : 1;  // V units per thread
   const uint8_t *pk, *pks;
-  uint8_t *kd, *vt, *sc;
+  uint8_t *vt, *sc;
   int k0, kend, tid, vu;
   bool full;
   float scale_log2;
-  uint32_t kx[kNK];
   uint32_t vx[8], pr[4];
   uint32_t kw, vw;
 
-  __device__ __forceinline__ void k_load(int i) {
-    const int u = tid + kPfWaves * 64 * i;
-    kx[i] = *reinterpret_cast<const uint32_t *>(pk + (u / kKDw) * Sh::kCell + 4 * (u % kKDw));
-  }
-  // K row kk: channel chunk c (8 channels in the order of the query operand) at 16 c
-  __device__ __forceinline__ void k_store(int i) {
-    const int u = tid + kPfWaves * 64 * i;
-    const int kk = u / kKDw, d = u % kKDw;
-    const uint32_t x = kx[i];
-    if constexpr (KFMT == QP_CODES_INT4) {
-      const uint32_t y = x >> 4;
-      *reinterpret_cast<u32x4_t *>(kd + kk * Sh::kKdRow + 16 * d) =
-          u32x4_t{nib_pair(x), nib_pair(y), nib_pair(x >> 8), nib_pair(y >> 8)};
-    } else {
-      *reinterpret_cast<u32x2_t *>(kd + kk * Sh::kKdRow + 8 * d) = i8_quad_bf16(x);
-    }
-  }
   // V unit u = (channel quad q4, K step ks, lane half h) = (u >> 2, (u >> 1) & 1, u & 1): the four channel rows of q4
   // at the 8 PV slots of (ks, h), i.e. keys slot_key(ks, h, 0..7). Unit j of the thread: tid + 256 j (mod HS).
   __device__ __forceinline__ void v_unit(int j) { vu = (tid + kPfWaves * 64 * j) & (HS - 1); }
@@ -148,14 +115,8 @@ struct WStager {
   __device__ __forceinline__ void s_store() {
     const int kk = tid & (kPfKeys - 1);
     const bool ok = full || k0 + kk < kend;
-    float a, e;
-    if constexpr (KFMT == QP_CODES_INT4) {
-      a = __uint_as_float(kw & 0xFFFFFFF0u) * scale_log2;
-      e = a * (float)(128u + (kw & 0xFu));
-    } else {
-      a = __uint_as_float(kw) * scale_log2;
-      e = a * 128.f;  // the operands are 128 + k
-    }
+    const float a = __uint_as_float(kw & 0xFFFFFFF0u) * scale_log2;
+    const float e = a * (float)(128u + (kw & 0xFu));
     const bool own = tid < kPfKeys;
     float *dummy = reinterpret_cast<float *>(sc + Sh::kScDummy);
     *(own ? reinterpret_cast<float *>(sc + Sh::kScA) + kk : dummy) = ok ? a : 0.f;
@@ -179,12 +140,6 @@ struct WStager {
   }
   // everything at once (the prologue's tiles)
   __device__ __forceinline__ void all() {
-    if constexpr (!Sh::kDirect) {
-#pragma unroll
-      for (int i = 0; i < kNK; ++i) k_load(i);
-#pragma unroll
-      for (int i = 0; i < kNK; ++i) k_store(i);
-    }
     v_all();
     s_load();
     s_store();
@@ -199,7 +154,7 @@ __device__ __forceinline__ bf16x8_t k_operand(uint32_t x) {
 
 // Rows of the wide kernel per wave and per workgroup: NT 32-row tiles per wave.
 template <int HS>
-constexpr int wide_nt() { return HS >= 256 ? 1 : 2; }  // at head 512 the 32 rows' query operands take 128 VGPRs
+constexpr int wide_nt() { return 1; }  // the 32 rows' query operands take 128 VGPRs
 
 template <int HS, int NT>
 struct WRows {
@@ -213,40 +168,17 @@ struct WRows {
   bool valid[NT];
 };
 
-// S^T += K Q^T of one 16-channel step for the row tiles, as inline assembly writing VGPRs. `last` adds 24 wait states:
-// a 16-pass XDL result is complete before anything reads it. WAIT puts 2 wait states before the MFMA, for a K operand
-// the VALU has just built (the compiler inserts them for its own MFMAs only).
-template <int NT, bool WAIT = false>
-__device__ __forceinline__ void wqk(f32x16_t (&s)[NT], bf16x8_t kop, const bf16x8_t (&q)[NT], bool first, bool last) {
-  if constexpr (WAIT) {
-    static_assert(NT == 1, "K operands built by the VALU: one row tile (head 512)");
-    if (first)
-      asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s[0]) : "v"(kop), "v"(q[0]));
-    else if (last)
-      asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
-                   : "+v"(s[0]) : "v"(kop), "v"(q[0]));
-    else
-      asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[0]) : "v"(kop), "v"(q[0]));
-  } else if constexpr (NT == 1) {
-    if (first)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s[0]) : "v"(kop), "v"(q[0]));
-    else if (last)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
-                   : "+v"(s[0]) : "v"(kop), "v"(q[0]));
-    else
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[0]) : "v"(kop), "v"(q[0]));
-  } else {
-    if (first)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, 0\n\tv_mfma_f32_32x32x16_bf16 %1, %2, %4, 0"
-                   : "=&v"(s[0]), "=&v"(s[1]) : "v"(kop), "v"(q[0]), "v"(q[1]));
-    else if (last)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, %0\n\tv_mfma_f32_32x32x16_bf16 %1, %2, %4, %1\n\t"
-                   "s_nop 7\n\ts_nop 7\n\ts_nop 7"
-                   : "+v"(s[0]), "+v"(s[1]) : "v"(kop), "v"(q[0]), "v"(q[1]));
-    else
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, %0\n\tv_mfma_f32_32x32x16_bf16 %1, %2, %4, %1"
-                   : "+v"(s[0]), "+v"(s[1]) : "v"(kop), "v"(q[0]), "v"(q[1]));
-  }
+// S^T += K Q^T of one 16-channel step, as inline assembly writing VGPRs. The 2 wait states before the MFMA are for a K
+// operand the VALU has just built (the compiler inserts them for its own MFMAs only); `last` adds 24 after it: a 16-pass
+// XDL result is complete before anything reads it.
+__device__ __forceinline__ void wqk(f32x16_t &s, bf16x8_t kop, bf16x8_t q, bool first, bool last) {
+  if (first)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(kop), "v"(q));
+  else if (last)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
+                 : "+v"(s) : "v"(kop), "v"(q));
+  else
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(kop), "v"(q));
 }
 
 // Softmax of one tile for the row tiles: scores from s (S^T), per-key scalars from the tile's scalar block sc; P16 in PV operand
@@ -320,11 +252,8 @@ __device__ __forceinline__ bool w_softmax(WRows<HS, NT> &r, const f32x16_t (&s)[
 template <int NT, int CT>
 __device__ __forceinline__ void wpv_step(f32x16_t (&acc)[NT][CT], int ct, bf16x8_t vop, const u32x4_t (&p)[NT][2],
                                          int ks) {
-  if constexpr (NT == 1)
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc[0][ct]) : "v"(vop), "v"(p[0][ks]));
-  else
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, %0\n\tv_mfma_f32_32x32x16_bf16 %1, %2, %4, %1"
-                 : "+a"(acc[0][ct]), "+a"(acc[1][ct]) : "v"(vop), "v"(p[0][ks]), "v"(p[1][ks]));
+  static_assert(NT == 1, "one row tile");
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc[0][ct]) : "v"(vop), "v"(p[0][ks]));
 }
 // Zeroes one accumulator tile with an MFMA on zero operands: as an assignment of zeros, the compiler kept one tile's
 // zeros in scratch across the restart loop at head 512 (all 256 AGPRs hold accumulators there). Only PV MFMAs, which
@@ -334,39 +263,6 @@ __device__ __forceinline__ void wzero(f32x16_t &acc) {
 }
 // 24 wait states: the last inline 32x32x16 MFMA's result (16 passes) is complete before anything else touches it
 __device__ __forceinline__ void wpv_drain() { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory"); }
-
-// Inverse rotation of one output row half in the O^T layout (lane half h holds channel 32 ct + 8 (i / 4) + 4 h + i % 4
-// at x[16 ct + i]): x <- ((x H) D) * scale, butterflies over the channel bits in ascending order (i % 4, then h across
-// lanes l ^ 32, then i / 4, then ct), as rht_kernel runs them on the same row.
-template <int HS>
-__device__ __forceinline__ void w_rotate_out(float (&x)[HS / 2], const float *signs, float scale, int h) {
-  constexpr int kE = HS / 2;
-  auto local = [&](int span) {
-#pragma unroll
-    for (int i = 0; i < kE; ++i)
-      if (!(i & span)) {
-        const float u = x[i], v = x[i + span];
-        x[i] = u + v;
-        x[i + span] = u - v;
-      }
-  };
-  local(1);  // channel bit 0
-  local(2);  // channel bit 1
-#pragma unroll
-  for (int i = 0; i < kE; ++i) {  // channel bit 2 = lane half
-    const float v = __shfl_xor(x[i], 32, 64);
-    x[i] = h ? v - x[i] : x[i] + v;
-  }
-  local(4);  // channel bit 3
-  local(8);  // channel bit 4
-#pragma unroll
-  for (int span = 16; span < kE; span <<= 1) local(span);  // channel bits 5.. = the channel tile
-#pragma unroll
-  for (int i = 0; i < kE; ++i) {
-    const int ch = 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3);
-    x[i] = x[i] * signs[ch] * scale;
-  }
-}
 
 template <int HS, int KFMT, bool SPAN, bool BS16>
 __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const PrefillParams p) {
@@ -460,16 +356,12 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
       else x = rv ? *reinterpret_cast<const u32x4_t *>(qr + Sh::step_chan(cs, h)) : u32x4_t{0u, 0u, 0u, 0u};
       qs += bf16_lo(x[0]) + bf16_hi(x[0]) + bf16_lo(x[1]) + bf16_hi(x[1]) + bf16_lo(x[2]) + bf16_hi(x[2]) +
             bf16_lo(x[3]) + bf16_hi(x[3]);
-      if constexpr (KFMT == QP_CODES_INT4) {  // K operand order per 8 channels: (c0, c4, c1, c5, c2, c6, c3, c7)
-        u32x4_t y;
-        y[0] = (x[0] & 0xFFFFu) | (x[2] << 16);
-        y[1] = (x[0] >> 16) | (x[2] & 0xFFFF0000u);
-        y[2] = (x[1] & 0xFFFFu) | (x[3] << 16);
-        y[3] = (x[1] >> 16) | (x[3] & 0xFFFF0000u);
-        r.qop[jt][cs] = as_bf16x8(y);
-      } else {
-        r.qop[jt][cs] = as_bf16x8(x);
-      }
+      u32x4_t y;  // K operand order per 8 channels: (c0, c4, c1, c5, c2, c6, c3, c7)
+      y[0] = (x[0] & 0xFFFFu) | (x[2] << 16);
+      y[1] = (x[0] >> 16) | (x[2] & 0xFFFF0000u);
+      y[2] = (x[1] & 0xFFFFu) | (x[3] << 16);
+      y[3] = (x[1] >> 16) | (x[3] & 0xFFFF0000u);
+      r.qop[jt][cs] = as_bf16x8(y);
     }
     qs += shfl_xor_f(qs, 32);
     r.qsum[jt] = qs;
@@ -484,13 +376,11 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
   const int ntiles = ke > kb ? (ke - kb + kPfKeys - 1) / kPfKeys : 0;
   const int vis_all = first_pos + 1;  // keys below this are visible to every row of the block
 
-  constexpr bool kDirect = Sh::kDirect;
   auto pk_of = [&](int t) { return smem + (t % Sh::kSlots) * Sh::kSlot; };
   const uint32_t lds0 = uniform((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem);
   auto pk_lds_of = [&](int t) { return lds0 + (uint32_t)((t % Sh::kSlots) * Sh::kSlot); };
-  auto kd_of = [&](int t) { return smem + Sh::kOffK + (t & 1) * Sh::kKd; };
   auto vb_of = [&](int t) { return smem + Sh::kOffV + (t % Sh::kVbufs) * Sh::kVb; };
-  auto sc_of = [&](int t) { return kDirect ? smem + Sh::kOffR + (t & 1) * Sh::kSc : vb_of(t) + Sh::kVt; };
+  auto sc_of = [&](int t) { return smem + Sh::kOffR + (t & 1) * Sh::kSc; };
   auto tile_key = [&](int t) { return kb + t * kPfKeys; };
   const PfCopies<Pf> copies(w, lane);
   const uint8_t *hbase = p.kcodes + (int64_t)kvh * p.ks2;
@@ -506,11 +396,10 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
       pf_gather<Pf>(p, trow, tile_key(t), ke, kvh, pk_of(t));
     }
   };
-  // the unpack of tile tv's codes and tile ts's scalars (the same tile unless K direct)
+  // the unpack of tile tv's values and tile ts's scalars
   auto stager = [&](int tv, int ts, bool full) {
     St st;
     st.pk = pk_of(tv);
-    st.kd = kd_of(tv);
     st.vt = vb_of(tv);
     st.pks = pk_of(ts);
     st.sc = sc_of(ts);
@@ -522,20 +411,13 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
     st.scale_log2 = p.scale_log2;
     return st;
   };
-  // S^T of tile t (K direct: lane half h reads code dwords 32 h + cs of key col, two steps per 8-byte read)
+  // S^T of tile t: lane half h reads code dwords 32 h + cs of key col, two steps per 8-byte read
   auto qk_tile = [&](f32x16_t (&sq)[NT], int t) {
     const uint8_t *kp = pk_of(t) + col * Sh::kCell + (HS / 4) * h;
-    const uint8_t *kr = kd_of(t) + col * Sh::kKdRow + 16 * h;
 #pragma unroll
-    for (int cs = 0; cs < HS / 16; ++cs) {
-      bf16x8_t q[NT];
-#pragma unroll
-      for (int jt = 0; jt < NT; ++jt) q[jt] = r.qop[jt][cs];
-      bf16x8_t kop;
-      if constexpr (kDirect) kop = k_operand(reinterpret_cast<const u32x2_t *>(kp)[cs >> 1][cs & 1]);
-      else kop = *reinterpret_cast<const bf16x8_t *>(kr + 32 * cs);
-      wqk<NT, kDirect>(sq, kop, q, cs == 0, cs == HS / 16 - 1);
-    }
+    for (int cs = 0; cs < HS / 16; ++cs)
+      wqk(sq[0], k_operand(reinterpret_cast<const u32x2_t *>(kp)[cs >> 1][cs & 1]), r.qop[0][cs], cs == 0,
+          cs == HS / 16 - 1);
   };
   if (tid == 0) restart_word = 0;
 
@@ -548,8 +430,8 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
 #pragma unroll
       for (int ct = 0; ct < HS / 32; ++ct) wzero(r.acc[jt][ct]);
     }
-    // ---- prologue: tiles 0..2 fetched, 0 and 1 unpacked (K direct: tile 0, and tile 1's scalars), tile 3 fetched,
-    // S(0), the first maximum, P(0)
+    // ---- prologue: tiles 0..2 fetched, tile 0 and tile 1's scalars unpacked, tile 3 fetched, S(0), the first maximum,
+    // P(0)
     fetch(0);
     if (ntiles > 1) fetch(1);
     if (ntiles > 2) fetch(2);
@@ -568,12 +450,8 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
     if (ntiles > 3) fetch(3);
     if (ntiles > 1) {
       St st = stager(1, 1, false);
-      if constexpr (kDirect) {
-        st.s_load();
-        st.s_store();
-      } else {
-        st.all();
-      }
+      st.s_load();
+      st.s_store();
     }
     f32x16_t s[NT];
     qk_tile(s, 0);
@@ -643,64 +521,33 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
           fetch(it + 4);
         }
       }
-      // ---- phase A: S^T of tile it + 1 beside the unpack of tile it + 2 (K direct: tile it + 1's V and tile it + 2's
-      // scalars); past the last tiles a stale slot goes into idle buffers, the same code path
-      St st = kDirect ? stager(it + 1, it + 2, kSteady) : stager(it + 2, it + 2, kSteady);
+      // ---- phase A: S^T of tile it + 1 beside the unpack of its V and of tile it + 2's scalars; past the last tiles a
+      // stale slot goes into idle buffers, the same code path
+      St st = stager(it + 1, it + 2, kSteady);
       f32x16_t sn[NT];
-      if constexpr (kDirect) {
-        const uint8_t *kp = pk_of(it + 1) + col * Sh::kCell + (HS / 4) * h;
-        constexpr int kCs = HS / 16;
-        u32x2_t kraw[2];  // code dword pairs j (steps 2 j, 2 j + 1) at kraw[j & 1], read two pairs ahead
-        kraw[0] = *reinterpret_cast<const u32x2_t *>(kp);
-        kraw[1] = *reinterpret_cast<const u32x2_t *>(kp + 8);
+      const uint8_t *kp = pk_of(it + 1) + col * Sh::kCell + (HS / 4) * h;
+      constexpr int kCs = HS / 16;
+      u32x2_t kraw[2];  // code dword pairs j (steps 2 j, 2 j + 1) at kraw[j & 1], read two pairs ahead
+      kraw[0] = *reinterpret_cast<const u32x2_t *>(kp);
+      kraw[1] = *reinterpret_cast<const u32x2_t *>(kp + 8);
 #pragma unroll
-        for (int cs = 0; cs < kCs; ++cs) {
-          const uint32_t x = kraw[(cs >> 1) & 1][cs & 1];
-          if ((cs & 1) && (cs >> 1) + 2 < kCs / 2)
-            kraw[(cs >> 1) & 1] = *reinterpret_cast<const u32x2_t *>(kp + 8 * ((cs >> 1) + 2));
-          bf16x8_t q[NT];
+      for (int cs = 0; cs < kCs; ++cs) {
+        const uint32_t x = kraw[(cs >> 1) & 1][cs & 1];
+        if ((cs & 1) && (cs >> 1) + 2 < kCs / 2)
+          kraw[(cs >> 1) & 1] = *reinterpret_cast<const u32x2_t *>(kp + 8 * ((cs >> 1) + 2));
+        wqk(sn[0], k_operand(x), r.qop[0][cs], cs == 0, cs == kCs - 1);
+        // the unpack, spread over the steps: the V units, then the scalars
 #pragma unroll
-          for (int jt = 0; jt < NT; ++jt) q[jt] = r.qop[jt][cs];
-          wqk<NT, true>(sn, k_operand(x), q, cs == 0, cs == kCs - 1);
-          // the unpack, spread over the steps: the V units, then the scalars
-#pragma unroll
-          for (int j = 0; j < St::kVUnits; ++j) {
-            const int b = 2 + 8 * j;
-            if (cs == b) { st.v_unit(j); st.v_load(0); st.v_load(1); }
-            if (cs == b + 1) { st.v_load(2); st.v_load(3); }
-            if (cs == b + 2) { st.v_perm(0); st.v_perm(1); st.v_perm(2); st.v_perm(3); }
-            if (cs == b + 3) { st.v_store(0); st.v_store(1); }
-            if (cs == b + 4) { st.v_store(2); st.v_store(3); }
-          }
-          if (cs == 2 + 8 * St::kVUnits) st.s_load();
-          if (cs == 4 + 8 * St::kVUnits) st.s_store();
+        for (int j = 0; j < St::kVUnits; ++j) {
+          const int b = 2 + 8 * j;
+          if (cs == b) { st.v_unit(j); st.v_load(0); st.v_load(1); }
+          if (cs == b + 1) { st.v_load(2); st.v_load(3); }
+          if (cs == b + 2) { st.v_perm(0); st.v_perm(1); st.v_perm(2); st.v_perm(3); }
+          if (cs == b + 3) { st.v_store(0); st.v_store(1); }
+          if (cs == b + 4) { st.v_store(2); st.v_store(3); }
         }
-      } else {
-        const uint8_t *kr = kd_of(it + 1) + col * Sh::kKdRow + 16 * h;
-        constexpr int kCs = HS / 16;
-        constexpr int kLag = St::kNK < 4 ? St::kNK : 4;
-        bf16x8_t kbuf[2];
-        kbuf[0] = *reinterpret_cast<const bf16x8_t *>(kr);
-        kbuf[1] = *reinterpret_cast<const bf16x8_t *>(kr + 32);
-#pragma unroll
-        for (int cs = 0; cs < kCs; ++cs) {
-          const bf16x8_t kop = kbuf[cs & 1];
-          if (cs + 2 < kCs) kbuf[cs & 1] = *reinterpret_cast<const bf16x8_t *>(kr + 32 * (cs + 2));
-          bf16x8_t q[NT];
-#pragma unroll
-          for (int jt = 0; jt < NT; ++jt) q[jt] = r.qop[jt][cs];
-          wqk<NT>(sn, kop, q, cs == 0, cs == kCs - 1);
-          // the unpack, spread over the steps
-          if (cs < St::kNK) st.k_load(cs);
-          if (cs >= kLag && cs < St::kNK + kLag) st.k_store(cs - kLag);
-          constexpr int b0 = St::kNK + kLag < kCs - 6 ? St::kNK + kLag : kCs - 6;
-          if (cs == b0) { st.v_load(0); st.v_load(1); }
-          if (cs == b0 + 1) { st.v_load(2); st.v_load(3); st.s_load(); }
-          if (cs == b0 + 2) { st.v_perm(0); st.v_perm(1); st.v_perm(2); st.v_perm(3); }
-          if (cs == b0 + 3) { st.v_store(0); st.v_store(1); }
-          if (cs == b0 + 4) { st.v_store(2); st.v_store(3); }
-          if (cs == b0 + 5) st.s_store();
-        }
+        if (cs == 2 + 8 * St::kVUnits) st.s_load();
+        if (cs == 4 + 8 * St::kVUnits) st.s_store();
       }
       // ---- phase B: O^T += V^T P^T of tile it beside the softmax of tile it + 1
       u32x4_t pn[NT][2];
@@ -771,30 +618,7 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
     const int rr = r0 + kRowsWave * w + 32 * jt + col;
     const int64_t tok = q0 + (valid ? rr / G : 0);
     const int64_t head = kvh * G + (valid ? rr % G : 0);
-    if constexpr (!kDirect) {  // K direct (head 512) always runs split (the merge rotates the 512-channel rows)
-      if (S == 1) {
-        const float inv = l > 0.f ? 1.f / l : 0.f;
-        uint16_t *orow = p.out + tok * p.os0 + head * p.os1;
-        float x[HS / 2];
-        // (l = 0: a row block without keys in its split, whose accumulators were never zeroed; the merge skips the
-        // partials of such blocks by their m = -inf, the only thing it reads of them)
-#pragma unroll
-        for (int ct = 0; ct < HS / 32; ++ct)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) x[16 * ct + i] = l > 0.f ? (r.acc[jt][ct][i] - csum) * inv : 0.f;
-        if (p.osigns) w_rotate_out<HS>(x, p.osigns, p.out_scale, h);
-        if (valid) {
-#pragma unroll
-          for (int ct = 0; ct < HS / 32; ++ct)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              *reinterpret_cast<u32x2_t *>(orow + 32 * ct + 8 * q + 4 * h) =
-                  u32x2_t{pack_bf16x2(x[16 * ct + 4 * q], x[16 * ct + 4 * q + 1]),
-                          pack_bf16x2(x[16 * ct + 4 * q + 2], x[16 * ct + 4 * q + 3])};
-        }
-        continue;
-      }
-    }
+    // (the kernel always runs split: the merge normalises and rotates the 512-channel rows)
     if (valid) {
       float *orow = p.so + tok * p.sos0 + head * p.sos1 + (int64_t)split * HS;
 #pragma unroll
@@ -821,18 +645,11 @@ void launch_wide(const PrefillParams &p, dim3 grid, bool span, hipStream_t s) {
   else prefill_wide_kernel<HS, KFMT, false, false><<<grid, kPfWaves * 64, 0, s>>>(p);
 }
 
-int prefill_wide_rows(int head_size) {
-  return head_size == 512 ? kPfWaves * 32 * wide_nt<512>() : kPfWaves * 32 * wide_nt<128>();
-}
+int prefill_wide_rows() { return kPfWaves * 32 * wide_nt<512>(); }
 
-// Heads 128 and 512 (with int4 keys): the router's choices (head 256 runs on the tile kernel at every GQA width).
-void prefill_wide(const PrefillParams &p, int head_size, int key_format, dim3 grid, bool span, hipStream_t s) {
-  if (head_size == 512) {
-    launch_wide<512, QP_CODES_INT4>(p, grid, span, s);
-  } else {
-    if (key_format == QP_CODES_INT4) launch_wide<128, QP_CODES_INT4>(p, grid, span, s);
-    else launch_wide<128, QP_CODES_INT8>(p, grid, span, s);
-  }
+// Head 512 with int4 keys.
+void prefill_wide(const PrefillParams &p, dim3 grid, bool span, hipStream_t s) {
+  launch_wide<512, QP_CODES_INT4>(p, grid, span, s);
 }
 
 }  // namespace qp

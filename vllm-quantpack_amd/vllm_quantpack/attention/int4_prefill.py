@@ -62,11 +62,10 @@ def prefill_attention(q, k_cache, v_cache, k_scale_cache, v_scale_cache, out, *,
     When the chunk alone cannot fill the GPU, the keys are split over workgroups
     (num_splits, 0 = automatic) and merged; the fp32 partials go to a workspace from torch's caching allocator.
     max_seqlen_k bounds the automatic split count; without it the block table's capacity stands in (no host sync).
-    Rows are (token, query head) pairs, so any GQA width fills the kernels' tiles. Head 128 from 8 query heads per KV
-    head, and head 512 with int4 keys, run the library's wide kernel (32x32x16 MFMAs; at head 512 always key-split, so
-    it takes a workspace); head 512 with int8
-    keys runs the split-KV decode kernel over causal query slices of the chunk and merges (the library picks the
-    path)."""
+    Rows are (token, query head) pairs, so any GQA width fills the kernels' tiles. Heads 64 and 128 run the library's
+    dual kernel (two waves per SIMD), head 256 its tile kernel, head 512 with int4 keys its wide kernel (always
+    key-split, so it takes a workspace); head 512 with int8 keys runs the split-KV decode kernel over causal query
+    slices of the chunk and merges (the library picks the path)."""
     cache, args = _prefill_args(q, k_cache, v_cache, k_scale_cache, v_scale_cache, out, cu_seqlens_q, seqused_k,
                                 block_table, max_seqlen_q, softmax_scale, max_seqlen_k, num_splits)
     args.rht_signs = _hip.ptr(rht_signs)
