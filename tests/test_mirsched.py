@@ -278,3 +278,41 @@ def test_pipeline_on_a_small_kernel(tmp_path):
                     str(tmp_path / "s.o")], check=True, capture_output=True)
     mfmas = lambda p: sum(1 for l in code(p) if l.startswith("v_mfma"))  # noqa: E731
     assert mfmas(tmp_path / "s.s") == mfmas(tmp_path / "direct.s") >= 2
+
+
+def test_loop_exits_that_read_an_inline_mfma_result_wait():
+    """A block after a loop that copies an accumulator tile right after the loop's last inline MFMA gets 18 wait states
+    at its start; the loop's own header, and an exit that touches other registers, get none. The build's scan follows
+    branches the same way: it flags the listing without the wait states and passes the one with them."""
+    import importlib.util
+    import os
+    import mirsched
+    spec = importlib.util.spec_from_file_location("qp_build", os.path.join(os.path.dirname(mirsched.__file__), "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    mfma = ('    INLINEASM &"v_mfma_f32_16x16x32_bf16 $0, $1, $2, $0", 1 /* sideeffect attdialect */, 10 /* regdef */, def '
+            '$agpr0_agpr1_agpr2_agpr3, 9 /* reguse */, $vgpr0_vgpr1_vgpr2_vgpr3, 9 /* reguse */, $vgpr4_vgpr5_vgpr6_vgpr7,'
+            ' 2147483657 /* reguse tiedto:$0 */, $agpr0_agpr1_agpr2_agpr3(tied-def 3)')
+
+    def function(exit_copy):
+        return "\n".join([
+            "---", "name:            kern", "body:             |", "  bb.0:", "    successors: %bb.1(0x80000000)", "",
+            "    S_NOP 0", "", "  bb.1:", "    successors: %bb.2(0x04000000), %bb.1(0x7c000000)", "", "    S_BARRIER", mfma,
+            "    S_CBRANCH_SCC1 %bb.1, implicit $scc", "", "  bb.2:", "    successors: %bb.3(0x80000000)", "",
+            "    S_BRANCH %bb.3", "", "  bb.3:", "", exit_copy, "    S_ENDPGM 0", "", "..."])
+
+    text, n = mirsched.schedule_mir(function("    $agpr8 = V_ACCVGPR_MOV_B32 $agpr2, implicit $exec"), "^kern")
+    assert n == 1
+    body = [l.strip() for l in text.split("\n")]
+    at = body.index("bb.2:")
+    assert [l for l in body[at + 1:] if l.startswith("S_")][:3] == ["S_NOP 7", "S_NOP 7", "S_NOP 1"]
+    assert text.count("S_NOP 7") == 2
+    other, _ = mirsched.schedule_mir(function("    $agpr8 = V_ACCVGPR_MOV_B32 $agpr9, implicit $exec"), "^kern")
+    assert "S_NOP 7" not in other
+
+    loop = ("kern:\n.LBB0_1:\n\ts_barrier\n;;#ASMSTART\n\tv_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3]\n;;#ASMEND\n"
+            "\ts_cbranch_scc1 .LBB0_3\n\ts_branch .LBB0_1\n.LBB0_2:\n\tv_accvgpr_mov_b32 a8, a2\n.LBB0_3:\n")
+    copy = "\tv_accvgpr_mov_b32 a8, a2\n\ts_endpgm\n"
+    assert [x[2] for x in build.mfma_hazards(loop + copy)] == ["v_accvgpr_mov_b32 a8, a2"]
+    assert build.mfma_hazards(loop + "\ts_nop 7\n\ts_nop 7\n\ts_nop 1\n" + copy) == []
+    assert build.mfma_hazards(loop + "\ts_endpgm\n") == []  # the copy in .LBB0_2 is on no path

@@ -123,10 +123,11 @@ def _compile(src, verbose):
 
 # Inline-assembly MFMAs are invisible to the compiler's hazard recognizer: it does not know that their results land
 # some cycles after issue, and may read them (a copy of its own, for instance) too early. The kernels place the
-# required wait states inside their assembly; this scan of the generated code checks that nothing reads or writes the
-# destination of an inline-assembly MFMA within MFMA_WAIT wait states (each intervening instruction counted as one,
-# s_nop N as N + 1), except a following MFMA that accumulates into exactly the same registers (srcC = vdst, which the
-# hardware orders). The compiler's own MFMAs are covered by its hazard recognizer.
+# required wait states inside their assembly, the scheduled build at the loop exits that need them (mirsched.py); this
+# scan of the generated code follows the control flow from every inline-assembly MFMA and checks that nothing reads or
+# writes its destination within MFMA_WAIT wait states (each intervening instruction counted as one, s_nop N as N + 1),
+# except a following MFMA that accumulates into exactly the same registers (srcC = vdst, which the hardware orders). The
+# compiler's own MFMAs are covered by its hazard recognizer.
 MFMA_WAIT = 18
 _REG = re.compile(r"\b([va])\[(\d+):(\d+)\]|\b([va])(\d+)\b")
 
@@ -144,8 +145,8 @@ def _vregs(text):
 
 def mfma_hazards(asm):
     """[(line, mfma, reader)] of too-early accesses to the results of inline-assembly MFMAs (those between the
-    compiler's ;;#ASMSTART / ;;#ASMEND markers) in one assembly listing."""
-    ins = []
+    compiler's ;;#ASMSTART / ;;#ASMEND markers) in one assembly listing, along every path of branches taken or not."""
+    ins, labels = [], {}
     inline = False
     for i, raw in enumerate(asm.splitlines()):
         l = raw.strip()
@@ -153,31 +154,46 @@ def mfma_hazards(asm):
             inline = True
         elif l.startswith(";;#ASMEND"):
             inline = False
+        elif raw.startswith(".LBB") and ":" in raw:
+            labels[raw.split(":")[0]] = len(ins)
         elif l and not l.startswith((";", ".")) and not raw.startswith((".", "_")):
             ins.append((i, l.split(";")[0].strip(), inline))
-    found = []
-    for k, (i, line, inl) in enumerate(ins):
-        if not (inl and line.startswith("v_mfma")):
-            continue
-        regs = _vregs(line.split(None, 1)[1].split(",")[0])
-        waits = 0
-        for _, nxt, _ in ins[k + 1:k + 1 + MFMA_WAIT]:
-            if waits >= MFMA_WAIT:
-                break
+
+    def access(k, regs, waits):
+        """The first too-early access from instruction k on, `waits` wait states after the MFMA."""
+        while k < len(ins) and waits < MFMA_WAIT:
+            nxt = ins[k][1]
             op = nxt.split()[0]
-            if op == "s_nop":
-                waits += int(nxt.split()[1]) + 1
-                continue
             args = nxt.split(None, 1)[1] if " " in nxt else ""
+            k += 1
+            if op == "s_nop":
+                waits += int(args) + 1
+                continue
+            waits += 1
+            if op.startswith("s_endpgm"):
+                return None
+            if op == "s_branch":
+                k = labels.get(args.strip(), len(ins))
+                continue
+            if op.startswith("s_cbranch"):
+                found = access(labels.get(args.strip(), len(ins)), regs, waits)
+                if found:
+                    return found
+                continue
             if op.startswith("v_mfma"):
                 ops = [a.strip() for a in args.split(",")]
                 if _vregs(ops[0]) == regs and _vregs(ops[3]) == regs and not regs & _vregs(",".join(ops[1:3])):
-                    waits += 1
                     continue
             if regs & _vregs(args):
-                found.append((i, line, nxt))
-                break
-            waits += 1
+                return nxt
+        return None
+
+    found = []
+    for k, (i, line, inl) in enumerate(ins):
+        if inl and line.startswith("v_mfma"):
+            reader = access(k + 1, _vregs(line.split(None, 1)[1].split(",")[0]), 0)
+            if reader:
+                found.append((i, line, reader))
     return found
 
 

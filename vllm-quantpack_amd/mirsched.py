@@ -25,13 +25,15 @@ remaining path whose operands are ready fills the issue slots. Dependences:
   * inline assembly reads EXEC (its vector instructions run under it, though the statement does not list it), so
     it never moves across an EXEC write such as a lane-masked region's s_and_saveexec;
   * a barrier (s_barrier) is a full fence: every instruction before it stays before it and every one after it stays
-    after it, register-only ones included. A variant that let the scalar add forming an LDS-DMA copy's M0 value move
-    from before a barrier to just after it gave results that differed from call to call (the cause was not found);
-    with the fence the prefill kernels measure the same;
+    after it, register-only ones included (the prefill kernels measure the same with this fence);
   * inline-assembly MFMAs (invisible to LLVM's hazard recognizer): one that carries trailing wait states stays after
     every earlier inline MFMA of its block, and no later one moves above it, so the wait states still follow the
     last of them;
   * a block's terminators stay at its end.
+Where a block that follows inline MFMAs (a loop's exit, where LLVM copies an accumulator tile to the registers the next
+loop has it in) accesses one of their results within 18 wait states, those wait states are put at its start. Without
+them the copy after a pair of the int8 keys' steady iterations read the last MFMA's tile two registers early, and the
+sum l of one row tile lost 2^-9 of a tile's share, in some calls and not in others.
 The build scans the final assembly for reads of inline-MFMA results within 18 wait states, VALU writes of MFMA
 sources within 2, and spills in MFMA loops, as for every other source.
 """
@@ -320,6 +322,45 @@ def _instructions(lines, h, j):
     return out
 
 
+MFMA_WAIT = 18  # wait states after which an inline MFMA's result can be accessed by anything else
+
+
+def _exit_waits(blocks):
+    """The blocks (by number) that need wait states at their start: `blocks` maps each block's number to (instructions,
+    successors), and a path from an inline MFMA into the block accesses its result within MFMA_WAIT wait states, other
+    than an MFMA that accumulates into it. Instructions count as one wait state each, S_NOP n as n + 1."""
+    need = set()
+
+    def waits(x):
+        if x.op == "S_NOP":
+            return int(x.text.split()[1]) + 1
+        return 1 + sum(int(n) + 1 for n in re.findall(r"s_nop\s+(\d+)", x.asm))
+
+    def walk(number, pending, first):
+        for x in blocks[number][0]:
+            hit = {u for u, left in pending.items() if left > 0 and u in (x.defs | x.uses)}
+            if hit and not (x.asm and x.mfmas):
+                need.add(first)
+                return
+            pending = {u: left - waits(x) for u, left in pending.items() if left > waits(x) and u not in hit}
+            if not pending:
+                return
+        for s in blocks[number][1]:
+            walk(s, pending, first)
+
+    for number, (insts, successors) in blocks.items():
+        pending = {}
+        for x in insts:
+            pending = {u: left - waits(x) for u, left in pending.items() if left > waits(x)}
+            if x.asm and x.mfmas:
+                left = MFMA_WAIT - sum(int(n) + 1 for n in re.findall(r"s_nop\s+(\d+)", x.asm.rsplit("v_mfma", 1)[1]))
+                pending.update({u: left for u in x.defs if left > 0})
+        if pending:
+            for s in successors:
+                walk(s, pending, s)
+    return need
+
+
 def schedule_mir(text, pattern):
     """The MIR text with every MFMA-holding block of the functions matching `pattern` rescheduled; returns (text,
     number of blocks rescheduled). Kill flags are dropped from moved blocks (the order they described changed)."""
@@ -327,16 +368,33 @@ def schedule_mir(text, pattern):
     # this point), and this LLVM's MIR parser rejects it when it names a stack object listed after it: drop it (the
     # round trip then reproduces LLVM's code exactly, spill code included).
     lines = [l for l in text.split("\n") if not re.match(r"^  scavengeFI:\s+'%stack\.\d+'\s*$", l)]
-    repl = []
+    repl, scheduled = [], 0
     for s, e in _function_ranges(lines, pattern):
+        blocks, where = {}, {}
         for h, j in _blocks(lines, s, e):
+            k = h - 1
+            successors = []
+            while not re.match(r"^  bb\.\d+", lines[k]):
+                if lines[k].startswith("    successors:"):
+                    successors = [int(n) for n in re.findall(r"%bb\.(\d+)", lines[k])]
+                k -= 1
+            number = int(re.match(r"^  bb\.(\d+)", lines[k]).group(1))
             insts = [Inst(t) for t in _instructions(lines, h, j)]
-            if not any(x.mfmas for x in insts):
+            if any(x.mfmas for x in insts):
+                insts = [Inst(re.sub(r"\bkilled ", "", x.text)) for x in schedule(insts)]
+                where[number] = (h, j)
+                scheduled += 1
+            blocks[number] = (insts, successors)
+            where.setdefault(number, (h, h))
+        need = _exit_waits(blocks)
+        for number, (h, j) in where.items():
+            if h == j and number not in need:
                 continue
-            repl.append((h, j, [re.sub(r"\bkilled ", "", x.text) for x in schedule(insts)]))
+            nops = ["    S_NOP 7", "    S_NOP 7", "    S_NOP 1"] if number in need else []
+            repl.append((h, j, nops + ([x.text for x in blocks[number][0]] + [""] if j > h else [])))
     for h, j, new in sorted(repl, reverse=True):
-        lines[h:j] = new + [""]
-    return "\n".join(lines), len(repl)
+        lines[h:j] = new
+    return "\n".join(lines), scheduled
 
 
 def main(argv=None):
