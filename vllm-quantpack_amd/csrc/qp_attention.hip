@@ -250,7 +250,7 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
   st = decode_routed(cache, &P.decode, route_row, 16, s);
   if (st != QP_OK) return st;
   const qp_merge_args m = merge_of(P.decode, a, cache->head_size);
-  return merge_routed(&m, row_tok, row_seq, P.rows_cap, nullptr, s);
+  return merge_routed(&m, row_tok, row_seq, P.rows_cap, nullptr, 0, s);
 }
 
 // ------------------------------------------------------------------------------ entry point without allocation

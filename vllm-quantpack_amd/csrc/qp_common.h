@@ -121,7 +121,7 @@ int slice_prefill(const qp_paged_cache *cache, const qp_prefill_args *a, const i
 int decode_routed(const qp_paged_cache *cache, const qp_decode_args *a, const int32_t *route_row, int max_rows,
                   hipStream_t s);
 int merge_routed(const qp_merge_args *a, const int32_t *row_tok, const int32_t *row_seq, int64_t rows,
-                 const int32_t *skip_seq, hipStream_t s);
+                 const int32_t *skip_seq, int min_keys, hipStream_t s);
 int prefill_run(const qp_paged_cache *cache, const qp_prefill_args *a, const int32_t *skip_seq, hipStream_t s);
 
 // Exact magic division for 0 <= x < 2^31 by d >= 2: m = ceil(2^(31+l) / d), l = ceil(log2 d);
@@ -278,6 +278,13 @@ __device__ __forceinline__ void load_query_row(uint32_t (&out)[E / 2], const uin
 // ------------------------------------------------------------------------------ shared kernel helpers
 
 namespace qp {
+
+// Keys per segment of a context of n keys cut into at most `segments` of them: whole 32-key chunks, and no fewer than
+// min_keys (0: no such floor). The kernels that write partials and the merge that reads them use the same rule;
+// segments that start at or past the context have nothing.
+__device__ __forceinline__ int segment_keys(int n, int segments, int min_keys) {
+  return max((n + segments * QP_DECODE_TILE - 1) / (segments * QP_DECODE_TILE) * QP_DECODE_TILE, min_keys);
+}
 
 __device__ __forceinline__ int fast_div(int x, uint32_t magic, uint32_t shift) {
   return (int)(__umulhi((uint32_t)x, magic) >> shift);

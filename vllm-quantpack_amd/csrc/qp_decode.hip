@@ -58,6 +58,7 @@ struct DecodeParams {
   float *ssum;
   int64_t sts0, sts1;
   int32_t num_q_heads, num_kv_heads, block_size, num_segments;
+  int32_t min_keys;             // floor of a segment's length (segment_keys)
   uint32_t bs_magic, bs_shift;  // pos / block_size == umulhi(pos, bs_magic) >> bs_shift for pos < 2^31
   float scale_log2;             // softmax_scale * log2(e)
   // Query slices (prefill through the split-KV kernel): when set, workgroup z takes slice z = (sequence, first token
@@ -117,7 +118,7 @@ __device__ __forceinline__ bool decode_work(const DecodeParams &p, int G, int h,
     nfull = d.n;
   }
   if (d.T <= 0 || nfull <= 0) return false;
-  const int seg = (nfull + p.num_segments * QP_DECODE_TILE - 1) / (p.num_segments * QP_DECODE_TILE) * QP_DECODE_TILE;
+  const int seg = segment_keys(nfull, p.num_segments, p.min_keys);
   d.kstart = seg_idx * seg;
   d.kend = min(d.n, d.kstart + seg);
   if (d.kstart < d.kend) return true;
@@ -1059,6 +1060,7 @@ struct MergeParams {
   int64_t sts0, sts1;
   const int32_t *cu_q, *used_k;
   int32_t num_seqs, num_segments, head_size;
+  int32_t min_keys;  // floor of a segment's length (segment_keys)
   uint16_t *out;
   int64_t os0, os1;
   float *lse;
@@ -1137,7 +1139,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     if (p.skip_seq && p.skip_seq[lo] >= 0) return;
   }
   const int n = p.used_k[lo];
-  const int seg = (n + p.num_segments * QP_DECODE_TILE - 1) / (p.num_segments * QP_DECODE_TILE) * QP_DECODE_TILE;
+  const int seg = segment_keys(n, p.num_segments, p.min_keys);
   const int active = seg > 0 ? min(p.num_segments, (n + seg - 1) / seg) : 0;
   const float *mrow = p.smax + (int64_t)srow * p.sts0 + (int64_t)head * p.sts1;
   const float *lrow = p.ssum + (int64_t)srow * p.sts0 + (int64_t)head * p.sts1;
@@ -1323,8 +1325,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
 // One wave per (row, query head), four rows per workgroup, for merges of few segments (the key splits of a prefill
 // chunk, decode batches of many sequences at 16 segments or fewer): every lane folds every segment of its channels
 // CPL l .. CPL l + CPL - 1 (head size 64 CPL), so no state is exchanged between lanes or waves. The row's statistics
-// are wave-uniform. Segments go in batches whose loads are all issued before any is used, past-context segments
-// loaded and ignored (as in merge_kernel). With signs the merged row is rotated back in registers (fwht_lanes).
+// are wave-uniform. Segments go in batches whose loads are all issued before any is used. With signs the merged row is rotated back in registers (fwht_lanes).
 template <bool RHT, int CPL>
 __global__ __launch_bounds__(256) void merge_wave_kernel(const MergeParams p, int rows) {
   const int lane = threadIdx.x & 63;
@@ -1334,7 +1335,7 @@ __global__ __launch_bounds__(256) void merge_wave_kernel(const MergeParams p, in
   int tok, seq;
   if (!merge_row_owner(p, srow, tok, seq)) return;
   const int n = p.used_k[seq];
-  const int seg = (n + p.num_segments * QP_DECODE_TILE - 1) / (p.num_segments * QP_DECODE_TILE) * QP_DECODE_TILE;
+  const int seg = segment_keys(n, p.num_segments, p.min_keys);
   const int active = seg > 0 ? min(p.num_segments, (n + seg - 1) / seg) : 0;
   const float *mrow = p.smax + (int64_t)srow * p.sts0 + (int64_t)head * p.sts1;
   const float *lrow = p.ssum + (int64_t)srow * p.sts0 + (int64_t)head * p.sts1;
@@ -1349,13 +1350,13 @@ __global__ __launch_bounds__(256) void merge_wave_kernel(const MergeParams p, in
   float a[CPL];
 #pragma unroll
   for (int i = 0; i < CPL; ++i) a[i] = 0.f;
-  for (int s0 = 0; s0 < p.num_segments; s0 += kBatch) {
+  for (int s0 = 0; s0 < active; s0 += kBatch) {
     float v[kBatch][CPL];
     float ms[kBatch], ls[kBatch];
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) {
       const int s = s0 + k;
-      if (s < p.num_segments) {
+      if (s < active) {
         load_channels<CPL>(orow + (int64_t)s * p.sos2, v[k]);
         ms[k] = mrow[s];
         ls[k] = lrow[s];
@@ -1366,9 +1367,6 @@ __global__ __launch_bounds__(256) void merge_wave_kernel(const MergeParams p, in
         ls[k] = 0.f;
       }
     }
-#pragma unroll
-    for (int k = 0; k < kBatch; ++k)
-      if (s0 + k >= active) ms[k] = -INFINITY;
     float bm = mt;
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) bm = fmaxf(bm, ms[k]);
@@ -1586,6 +1584,7 @@ void decode_params(const qp_paged_cache *cache, const qp_decode_args *a, DecodeP
   p.sts1 = a->segm_stat_stride[1];
   p.num_q_heads = a->num_q_heads;
   p.num_segments = a->num_segments;
+  p.min_keys = 0;
   p.scale_log2 = a->softmax_scale * kLog2e;
   p.slices = nullptr;
   p.tok_group = 0;
@@ -1608,6 +1607,7 @@ MergeParams merge_params(const qp_merge_args *a) {
   p.used_k = a->seqused_k;
   p.num_seqs = a->num_seqs;
   p.num_segments = a->num_segments;
+  p.min_keys = 0;
   p.head_size = a->head_size;
   p.out = static_cast<uint16_t *>(a->out);
   p.os0 = a->out_stride[0];
@@ -1733,10 +1733,11 @@ int decode_routed(const qp_paged_cache *cache, const qp_decode_args *a, const in
 // (row_tok[r] < 0: unused). With skip_seq and no row maps, a plain merge over the tokens leaves the sequences with
 // skip_seq[i] >= 0 alone.
 int merge_routed(const qp_merge_args *a, const int32_t *row_tok, const int32_t *row_seq, int64_t rows,
-                 const int32_t *skip_seq, hipStream_t s) {
+                 const int32_t *skip_seq, int min_keys, hipStream_t s) {
   const int st = check_merge(a);
   if (st != QP_OK) return st;
   MergeParams p = merge_params(a);
+  p.min_keys = min_keys;
   p.row_tok = row_tok;
   p.row_seq = row_seq;
   p.skip_seq = skip_seq;
@@ -1831,6 +1832,7 @@ int slice_prefill(const qp_paged_cache *cache, const qp_prefill_args *a, const i
   p.sts0 = (int64_t)a->num_q_heads * L.segments;
   p.num_q_heads = a->num_q_heads;
   p.num_segments = L.segments;
+  p.min_keys = 0;
   p.scale_log2 = a->softmax_scale * kLog2e;
   p.slices = slices;
   p.tok_group = 0;
@@ -1862,7 +1864,7 @@ int slice_prefill(const qp_paged_cache *cache, const qp_prefill_args *a, const i
   m.out_stride[1] = a->out_stride[1];
   m.rht_signs = a->rht_signs;
   m.rht_out_scale = a->rht_out_scale;
-  return merge_routed(&m, nullptr, nullptr, 0, skip_seq, s);
+  return merge_routed(&m, nullptr, nullptr, 0, skip_seq, 0, s);
 }
 
 }  // namespace qp

@@ -27,6 +27,7 @@ struct PrefillParams {
   float *smax, *ssum;
   int64_t sos0, sos1, sts0, sts1;
   int32_t num_seqs, num_q_heads, num_kv_heads, block_size, num_splits;
+  int32_t min_keys;        // floor of a key split's length (segment_keys)
   uint32_t bs_magic, bs_shift;
   float scale_log2;
   const float *qsigns;     // forward rotation of the query rows as they load (null: q in the cache's domain)

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
   const int kend = max(0, min(n, n - qlen + t_last + 1));  // keys any row of the block can see
   // key split: the split-KV segment rule shared with qp_merge_segments
   const int S = p.num_splits;
-  const int seg = (n + S * QP_DECODE_TILE - 1) / (S * QP_DECODE_TILE) * QP_DECODE_TILE;
+  const int seg = segment_keys(n, S, p.min_keys);
   const int kb = split * seg;
   const int ke = uniform(min(kend, kb + seg));
   if (S > 1 && kb >= n) return;  // inactive segment: the merge does not read it

@@ -301,7 +301,7 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
   const int first_pos = n - qlen + t_first;
   const int kend = max(0, min(n, n - qlen + t_last + 1));  // keys any row of the block can see
   const int S = p.num_splits;
-  const int seg = (n + S * QP_DECODE_TILE - 1) / (S * QP_DECODE_TILE) * QP_DECODE_TILE;
+  const int seg = segment_keys(n, S, p.min_keys);
   const int kb = split * seg;
   const int ke = uniform(min(kend, kb + seg));
   if (S > 1 && kb >= n) return;  // inactive segment: the merge does not read it
