@@ -10,9 +10,15 @@
 // (x -> x D H, Sylvester H, +/-1 diagonal D) in fp32 and rounded to bf16, as `single_rht(x.float()).to(x.dtype)`
 // (k8v4_kv.py:71-72).
 //
-// One wave per (token, KV head): lane l owns channels l*E .. l*E + E - 1 (E = head_size / 64), reductions are wave
-// shuffles and the rotation is an in-register fast Walsh-Hadamard transform.
+// A lane owns 8 consecutive channels, so a row is held by 8 to 64 lanes and a workgroup stores 4 to 32 consecutive tokens
+// of one KV head (adjacent cells where slots are). Three stages of the Walsh-Hadamard transform are then local to a
+// lane and the others, like the reductions, are DPP moves and row swaps on the VALU; a lane loads its 16 bytes of a row
+// at once and stores its int4 codes as one dword. With one wave per (token, head), 2 channels per lane, LDS permutes for
+// every exchange and 64-bit divisions for the slot, 4096 tokens of 8 heads of 128 (21 MB) took 22 us;
+// this takes 11.2-11.6, set by the VALU work of the rotation and the quantiser's divisions as much as by memory.
 #include "qp_common.h"
+
+#include <type_traits>
 
 namespace qp {
 
@@ -31,96 +37,199 @@ struct StoreParams {
   uint32_t *vwords;
   int64_t vws0, vws1, vws2;
   int32_t num_tokens, block_size;
+  uint32_t bs_magic, bs_shift;  // slot / block_size == fast_div(slot, ...) for slots below 2^31 and block_size > 1
   const float *signs;
 };
 
 __device__ __forceinline__ float round_half_away(float x) { return x >= 0.f ? truncf(x + 0.5f) : truncf(x - 0.5f); }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-  return v;
-}
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v = fminf(v, __shfl_xor(v, m, 64));
-  return v;
+constexpr int kStoreThreads = 256;
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
-template <int E>
-__device__ __forceinline__ void load_row(float (&x)[E], const uint16_t *row, const float *signs, int lane) {
-#pragma unroll
-  for (int i = 0; i < E; ++i) x[i] = __uint_as_float((uint32_t)row[lane * E + i] << 16);
-  if (signs) {
-#pragma unroll
-    for (int i = 0; i < E; ++i) x[i] *= signs[lane * E + i];
-    fwht_wave<E>(x, lane);
-#pragma unroll
-    for (int i = 0; i < E; ++i) x[i] = __uint_as_float((uint32_t)f32_to_bf16_bits(x[i]) << 16);
+// The butterfly of the Walsh-Hadamard transform over lane bit M: the lower lane gets lower + upper, the upper one lower -
+// upper. sign: -1 in upper lanes, +1 in lower ones (the product is exact, so the fma rounds once, as the sum does).
+template <int M>
+__device__ __forceinline__ float lane_butterfly(float x, float sign) {
+  if constexpr (M == 1) {
+    return fmaf(x, sign, dpp<0xB1>(x));  // quad_perm (1, 0, 3, 2)
+  } else if constexpr (M == 2) {
+    return fmaf(x, sign, dpp<0x4E>(x));  // quad_perm (2, 3, 0, 1)
+  } else if constexpr (M == 4) {
+    return fmaf(x, sign, dpp<0x1B>(dpp<0x141>(x)));  // row_half_mirror (l ^ 7), then quad_perm (3, 2, 1, 0) (l ^ 3)
+  } else if constexpr (M == 8) {
+    return fmaf(x, sign, dpp<0x128>(x));  // row_ror 8
+  } else {  // a row (half) swap gives both lanes of a pair the lower and the upper value
+    const uint32_t b = __float_as_uint(x);
+    const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(b, b, false, false)
+                           : __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return fmaf(__uint_as_float(r[1]), sign, __uint_as_float(r[0]));
   }
 }
 
-// Asymmetric int4 of the wave's row: packs this lane's E channels into E/2 bytes, returns the word.
-template <int E>
-__device__ __forceinline__ uint32_t quant_int4(const float (&x)[E], uint8_t *codes_row, int lane) {
+// Maximum over the LANES lanes of a row, every lane receiving it (a group's lanes agree after each step, so mirrors serve
+// as exchanges).
+template <int LANES>
+__device__ __forceinline__ float row_max(float v) {
+  v = fmaxf(v, dpp<0xB1>(v));
+  v = fmaxf(v, dpp<0x4E>(v));
+  v = fmaxf(v, dpp<0x141>(v));
+  if constexpr (LANES >= 16) v = fmaxf(v, dpp<0x140>(v));  // row_mirror
+  if constexpr (LANES >= 32) {
+    const uint32_t b = __float_as_uint(v);
+    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  if constexpr (LANES >= 64) {
+    const uint32_t b = __float_as_uint(v);
+    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  return v;
+}
+
+// The lane's 8 channels of a row as bf16 pairs.
+template <bool VEC>
+__device__ __forceinline__ u32x4_t load_bf16x8(const uint16_t *row) {
+  if constexpr (VEC) {
+    return *reinterpret_cast<const u32x4_t *>(row);
+  } else {
+    u32x4_t v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (uint32_t)row[2 * i] | ((uint32_t)row[2 * i + 1] << 16);
+    return v;
+  }
+}
+
+// fp32 channels of the row, rotated and rounded to bf16 when ROT: (x D) H, butterflies over channel bits in ascending
+// order as rht_kernel runs them.
+template <int LANES, bool ROT>
+__device__ __forceinline__ void store_row(float (&x)[8], u32x4_t v, const float (&signs)[8], int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[2 * i] = bf16_lo(v[i]);
+    x[2 * i + 1] = bf16_hi(v[i]);
+  }
+  if constexpr (ROT) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] *= signs[i];
+#pragma unroll
+    for (int span = 1; span < 8; span <<= 1)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (!(i & span)) {
+          const float a = x[i], b = x[i + span];
+          x[i] = a + b;
+          x[i + span] = a - b;
+        }
+    auto stage = [&](auto tag) {
+      constexpr int M = decltype(tag)::value;
+      if constexpr (M < LANES) {
+        const float sign = (lane & M) ? -1.f : 1.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = lane_butterfly<M>(x[i], sign);
+      }
+    };
+    stage(std::integral_constant<int, 1>{});
+    stage(std::integral_constant<int, 2>{});
+    stage(std::integral_constant<int, 4>{});
+    stage(std::integral_constant<int, 8>{});
+    stage(std::integral_constant<int, 16>{});
+    stage(std::integral_constant<int, 32>{});
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = __uint_as_float((uint32_t)f32_to_bf16_bits(x[i]) << 16);
+  }
+}
+
+// N code dwords of the lane to its place in the row.
+template <bool VEC, int N>
+__device__ __forceinline__ void put_codes(uint8_t *dst, const uint32_t (&w)[N]) {
+  if constexpr (VEC) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) reinterpret_cast<uint32_t *>(dst)[i] = w[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4 * N; ++i) dst[i] = (uint8_t)(w[i / 4] >> (8 * (i % 4)));
+  }
+}
+
+// Asymmetric int4 of a row: stores the lane's 8 codes as 4 bytes, returns the word.
+template <int LANES, bool VEC>
+__device__ __forceinline__ uint32_t quant_int4(const float (&x)[8], uint8_t *codes_row, int lane) {
   float lo = x[0], hi = x[0];
 #pragma unroll
-  for (int i = 1; i < E; ++i) {
+  for (int i = 1; i < 8; ++i) {
     lo = fminf(lo, x[i]);
     hi = fmaxf(hi, x[i]);
   }
-  lo = wave_min(lo);
-  hi = wave_max(hi);
+  lo = -row_max<LANES>(-lo);
+  hi = row_max<LANES>(hi);
   const float scale = fmaxf((hi - lo) / 15.0f, 1e-6f);
   const float zp = fminf(fmaxf(round_half_away(-lo / scale), 0.f), 15.f);
   const float inv = 1.0f / scale;
-  if constexpr (E == 1) {
-    // head 64, one channel per lane: the byte of channels 2i and 2i + 1 joins lanes 2i and 2i + 1
-    const uint32_t q = (uint32_t)fminf(fmaxf(round_half_away(fmaf(x[0], inv, zp)), 0.f), 15.f);
-    const uint32_t qn = (uint32_t)__shfl_xor((int)q, 1, 64);
-    if (!(lane & 1)) codes_row[lane >> 1] = (uint8_t)((q & 0xF) | ((qn & 0xF) << 4));
-  } else {
-    uint8_t b[E / 2];
+  uint32_t w[1] = {0};
 #pragma unroll
-    for (int i = 0; i < E; i += 2) {
-      const uint32_t q0 = (uint32_t)fminf(fmaxf(round_half_away(fmaf(x[i], inv, zp)), 0.f), 15.f);
-      const uint32_t q1 = (uint32_t)fminf(fmaxf(round_half_away(fmaf(x[i + 1], inv, zp)), 0.f), 15.f);
-      b[i / 2] = (uint8_t)((q0 & 0xF) | ((q1 & 0xF) << 4));
-    }
-#pragma unroll
-    for (int i = 0; i < E / 2; ++i) codes_row[lane * (E / 2) + i] = b[i];
+  for (int i = 0; i < 8; ++i) {
+    // clamp(round_half_away(y), 0, 15): a negative y rounds to 0 at most, so only y + 0.5 of the others is truncated
+    const float y = fmaf(x[i], inv, zp);
+    w[0] |= (uint32_t)fminf(fmaxf(y, 0.f) + 0.5f, 15.f) << (4 * i);
   }
+  put_codes<VEC>(codes_row + 4 * lane, w);
   return (__float_as_uint(scale) & 0xFFFFFFF0u) | (uint32_t)zp;
 }
 
-template <int E>
-__device__ __forceinline__ uint32_t quant_int8(const float (&x)[E], uint8_t *codes_row, int lane) {
+template <int LANES, bool VEC>
+__device__ __forceinline__ uint32_t quant_int8(const float (&x)[8], uint8_t *codes_row, int lane) {
   float a = fabsf(x[0]);
 #pragma unroll
-  for (int i = 1; i < E; ++i) a = fmaxf(a, fabsf(x[i]));
-  a = wave_max(a);
+  for (int i = 1; i < 8; ++i) a = fmaxf(a, fabsf(x[i]));
+  a = row_max<LANES>(a);
   const float scale = fmaxf(a / 127.0f, 1e-6f);
+  uint32_t w[2] = {0, 0};
 #pragma unroll
-  for (int i = 0; i < E; ++i) {
+  for (int i = 0; i < 8; ++i) {
     const float q = fminf(fmaxf(round_half_away(x[i] / scale), -127.f), 127.f);
-    codes_row[lane * E + i] = (uint8_t)(int8_t)q;
+    w[i / 4] |= (uint32_t)(uint8_t)(int8_t)q << (8 * (i % 4));
   }
+  put_codes<VEC>(codes_row + 8 * lane, w);
   return __float_as_uint(scale);
 }
 
-template <int E, int KFMT>
-__global__ __launch_bounds__(64) void store_kernel(const StoreParams p) {
-  const int tok = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+// VEC: rows of 16-byte aligned bf16 and 4-byte aligned codes (the host checks); else element by element.
+template <int HS, int KFMT, bool VEC, bool ROT>
+__global__ __launch_bounds__(kStoreThreads) void store_kernel(const StoreParams p) {
+  constexpr int LANES = HS / 8;
+  const int lane = threadIdx.x % LANES, h = blockIdx.y;
+  const int64_t tok = (int64_t)blockIdx.x * (kStoreThreads / LANES) + threadIdx.x / LANES;
+  if (tok >= p.num_tokens) return;
+  const u32x4_t kv = load_bf16x8<VEC>(p.key + tok * p.kst0 + h * p.kst1 + 8 * lane);
+  const u32x4_t vv = load_bf16x8<VEC>(p.value + tok * p.vst0 + h * p.vst1 + 8 * lane);
   const int64_t slot = p.slots[tok];
+  float signs[8];
+  if constexpr (ROT) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) signs[i] = p.signs[8 * lane + i];
+  }
   if (slot < 0) return;
-  const int64_t blk = slot / p.block_size, off = slot % p.block_size;
-  float x[E];
-  load_row<E>(x, p.key + tok * p.kst0 + h * p.kst1, p.signs, lane);
+  int64_t blk, off;
+  if ((slot >> 31) == 0 && p.block_size > 1) {
+    blk = fast_div((int)slot, p.bs_magic, p.bs_shift);
+    off = slot - blk * p.block_size;
+  } else {
+    blk = slot / p.block_size;
+    off = slot % p.block_size;
+  }
+  float x[8];
+  store_row<LANES, ROT>(x, kv, signs, lane);
   uint8_t *krow = p.kcodes + blk * p.ks0 + off * p.ks1 + h * p.ks2;
-  const uint32_t kw = KFMT == QP_CODES_INT4 ? quant_int4<E>(x, krow, lane) : quant_int8<E>(x, krow, lane);
-  load_row<E>(x, p.value + tok * p.vst0 + h * p.vst1, p.signs, lane);
+  const uint32_t kw =
+      KFMT == QP_CODES_INT4 ? quant_int4<LANES, VEC>(x, krow, lane) : quant_int8<LANES, VEC>(x, krow, lane);
+  store_row<LANES, ROT>(x, vv, signs, lane);
   uint8_t *vrow = p.vcodes + blk * p.vs0 + off * p.vs1 + h * p.vs2;
-  const uint32_t vw = quant_int4<E>(x, vrow, lane);
+  const uint32_t vw = quant_int4<LANES, VEC>(x, vrow, lane);
   if (lane == 0) {
     p.kwords[blk * p.kws0 + off * p.kws1 + h * p.kws2] = kw;
     p.vwords[blk * p.vws0 + off * p.vws1 + h * p.vws2] = vw;
@@ -174,10 +283,23 @@ using namespace qp;
 
 namespace {
 
-template <int E>
-void launch_store(const StoreParams &p, int kfmt, dim3 grid, hipStream_t s) {
-  if (kfmt == QP_CODES_INT4) store_kernel<E, QP_CODES_INT4><<<grid, 64, 0, s>>>(p);
-  else store_kernel<E, QP_CODES_INT8><<<grid, 64, 0, s>>>(p);
+template <int HS, int KFMT>
+void launch_store_format(const StoreParams &p, dim3 grid, bool vec, hipStream_t s) {
+  if (p.signs) {
+    if (vec) store_kernel<HS, KFMT, true, true><<<grid, kStoreThreads, 0, s>>>(p);
+    else store_kernel<HS, KFMT, false, true><<<grid, kStoreThreads, 0, s>>>(p);
+  } else {
+    if (vec) store_kernel<HS, KFMT, true, false><<<grid, kStoreThreads, 0, s>>>(p);
+    else store_kernel<HS, KFMT, false, false><<<grid, kStoreThreads, 0, s>>>(p);
+  }
+}
+
+template <int HS>
+void launch_store(const StoreParams &p, int kfmt, int num_kv_heads, bool vec, hipStream_t s) {
+  constexpr int kTokens = kStoreThreads / (HS / 8);  // per workgroup
+  const dim3 grid((p.num_tokens + (int64_t)kTokens - 1) / kTokens, num_kv_heads);
+  if (kfmt == QP_CODES_INT4) launch_store_format<HS, QP_CODES_INT4>(p, grid, vec, s);
+  else launch_store_format<HS, QP_CODES_INT8>(p, grid, vec, s);
 }
 
 template <int E>
@@ -224,14 +346,20 @@ extern "C" int qp_store(const qp_paged_cache *cache, const qp_store_args *a, qp_
   p.vws2 = cache->value.word_stride[2];
   p.num_tokens = a->num_tokens;
   p.block_size = cache->block_size;
+  p.bs_magic = p.bs_shift = 0;
+  if (p.block_size > 1) div_magic((uint32_t)p.block_size, &p.bs_magic, &p.bs_shift);
   p.signs = a->rht_signs;
-  const dim3 grid(a->num_tokens, cache->num_kv_heads);
+  // vector accesses where every row allows them; views of any alignment go element by element
+  bool vec = aligned(p.key, 16) && aligned(p.value, 16) && aligned(p.kcodes, 4) && aligned(p.vcodes, 4);
+  for (int i = 0; i < 2; ++i) vec = vec && a->key_stride[i] % 8 == 0 && a->value_stride[i] % 8 == 0;
+  for (int i = 0; i < 3; ++i) vec = vec && cache->key.code_stride[i] % 4 == 0 && cache->value.code_stride[i] % 4 == 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int nkv = cache->num_kv_heads;
   switch (hs) {
-    case 64: launch_store<1>(p, cache->key.format, grid, s); break;
-    case 128: launch_store<2>(p, cache->key.format, grid, s); break;
-    case 256: launch_store<4>(p, cache->key.format, grid, s); break;
-    default: launch_store<8>(p, cache->key.format, grid, s); break;
+    case 64: launch_store<64>(p, cache->key.format, nkv, vec, s); break;
+    case 128: launch_store<128>(p, cache->key.format, nkv, vec, s); break;
+    case 256: launch_store<256>(p, cache->key.format, nkv, vec, s); break;
+    default: launch_store<512>(p, cache->key.format, nkv, vec, s); break;
   }
   return launch_status();
 }
