@@ -554,8 +554,9 @@ __device__ __forceinline__ void finish_workgroup(WaveState<HS, KFMT, NCT> &st, u
 // The same merge without waiting for the slowest wave before parking: every wave parks its unscaled rows (acc - c) in
 // its own stage buffers (REGION bytes from smem + w * REGION, free once its last chunk is read) as soon as its loop
 // ends, while the other waves still run; after one barrier all threads sum the parked rows with the factors
-// 2^(m_w - M). Only valid rows are parked. st_m / st_l: WAVES * NCT * 16 floats each, outside the stage buffers.
-template <int HS, int KFMT, int NCT, int WAVES, int REGION>
+// 2^(m_w - M). Only valid rows are parked. st_m / st_l: a wave's NCT * 16 maxima and sums, STRIDE floats from one wave to
+// the next, outside the stage buffers.
+template <int HS, int KFMT, int NCT, int WAVES, int REGION, int STRIDE>
 __device__ __forceinline__ void finish_workgroup_own(WaveState<HS, KFMT, NCT> &st, uint8_t *smem, float *st_m,
                                                      float *st_l, const DecodeParams &p, int w, int col, int g,
                                                      int row0, int T, int G, int h, int seg_idx) {
@@ -571,8 +572,8 @@ __device__ __forceinline__ void finish_workgroup_own(WaveState<HS, KFMT, NCT> &s
   if (g == 0) {
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) {
-      st_m[w * kRows + ct * 16 + col] = st.m[ct];
-      st_l[w * kRows + ct * 16 + col] = st.l[ct];
+      st_m[w * STRIDE + ct * 16 + col] = st.m[ct];
+      st_l[w * STRIDE + ct * 16 + col] = st.l[ct];
     }
   }
   float *own = reinterpret_cast<float *>(smem + w * REGION);
@@ -600,11 +601,11 @@ __device__ __forceinline__ void finish_workgroup_own(WaveState<HS, KFMT, NCT> &s
     const int r = idx / (HS / 4), c4 = idx % (HS / 4);
     float M = -INFINITY;
 #pragma unroll
-    for (int ww = 0; ww < WAVES; ++ww) M = fmaxf(M, st_m[ww * kRows + r]);
+    for (int ww = 0; ww < WAVES; ++ww) M = fmaxf(M, st_m[ww * STRIDE + r]);
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int ww = 0; ww < WAVES; ++ww) {
-      const float mw = st_m[ww * kRows + r];
+      const float mw = st_m[ww * STRIDE + r];
       const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
       const float4 v = reinterpret_cast<const float4 *>(smem + ww * REGION)[r * (kORow / 4) + c4];
       sum.x = fmaf(v.x, f, sum.x);
@@ -623,11 +624,11 @@ __device__ __forceinline__ void finish_workgroup_own(WaveState<HS, KFMT, NCT> &s
       if (r < R) {
         float M = -INFINITY, L = 0.f;
 #pragma unroll
-        for (int ww = 0; ww < WAVES; ++ww) M = fmaxf(M, st_m[ww * kRows + r]);
+        for (int ww = 0; ww < WAVES; ++ww) M = fmaxf(M, st_m[ww * STRIDE + r]);
 #pragma unroll
         for (int ww = 0; ww < WAVES; ++ww) {
-          const float mw = st_m[ww * kRows + r];
-          if (mw != -INFINITY) L += st_l[ww * kRows + r] * __builtin_amdgcn_exp2f(mw - M);
+          const float mw = st_m[ww * STRIDE + r];
+          if (mw != -INFINITY) L += st_l[ww * STRIDE + r] * __builtin_amdgcn_exp2f(mw - M);
         }
         const int t = r / G, j = r % G;
         const int64_t o = (int64_t)(row0 + t) * p.sts0 + (int64_t)(h * G + j) * p.sts1 + seg_idx;
@@ -937,7 +938,10 @@ __global__ __launch_bounds__(WAVES * 64) void decode_span_kernel(const DecodePar
   __shared__ __attribute__((aligned(16))) float4 kfl[WAVES][kStages][kChunk];
   // the merge parks each wave's rows in its own stage buffers where they fit (finish_workgroup_own)
   constexpr bool kOwnMerge = NCT * 16 * (HS + 4) * 4 <= kStages * 2 * Sh::kHalf;
-  __shared__ float mst[2][kOwnMerge ? WAVES * NCT * 16 : 1];
+  // (its row statistics go to the wave's own scalars, free like its stages once its last chunk is read: with 83 KB the
+  // workgroup at head 128 would be one too large for two of them on a CU)
+  constexpr int kFlStride = kStages * kChunk * 4;  // floats of a wave's scalars
+  static_assert(!kOwnMerge || 2 * NCT * 16 <= kFlStride, "row statistics in the wave's scalars");
   __shared__ f32x4_t rsc[WAVES][acc_in_agprs<HS, KFMT, NCT>() ? 64 : 1];  // rescale of AGPR accumulators
   // Rotated query rows (rotate_rows_shared): their own buffer at one row tile; with two the stage cells hold them until
   // every wave has read its operands (one more barrier before the first copies).
@@ -1045,8 +1049,8 @@ __global__ __launch_bounds__(WAVES * 64) void decode_span_kernel(const DecodePar
     }
   }
   if constexpr (kOwnMerge)
-    finish_workgroup_own<HS, KFMT, NCT, WAVES, kStages * 2 * Sh::kHalf>(st, smem, mst[0], mst[1], p, w, col, g, row0, T,
-                                                                        G, h, seg_idx);
+    finish_workgroup_own<HS, KFMT, NCT, WAVES, kStages * 2 * Sh::kHalf, kFlStride>(
+        st, smem, &kfl[0][0][0].x, &kfl[0][0][0].x + NCT * 16, p, w, col, g, row0, T, G, h, seg_idx);
   else if constexpr (kParMerge) finish_workgroup<HS, KFMT, NCT, WAVES>(st, smem, p, w, col, g, row0, T, G, h, seg_idx);
   else finish_workgroup_serial<HS, KFMT, NCT, WAVES>(st, smem, p, w, col, g, row0, T, G, h, seg_idx);
 }
