@@ -70,6 +70,7 @@ struct AttentionPlan {
   bool routed;        // a route table splits the batch between decode and prefill
   int rows_cap;       // segment-buffer rows the route table hands out
   int64_t off_route, off_tok, off_seq, off_segm, off_prefill, total;
+  int min_keys;       // floor of a segment's length
   int64_t segm_rows;  // rows of split-KV partials in the workspace (0: the caller's segment buffers hold them)
   qp_prefill_args prefill;
   qp_decode_args decode;
@@ -161,6 +162,13 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
   d.segm_stat_stride[1] = a->segm_stat_stride[1];
   d.segm_rows = a->segm_rows;
   d.query_signs = a->rht_signs;
+  // In mixed batches that fill the device with workgroups, segments have at least 512 keys (two 32-key chunks for each
+  // of a workgroup's 8 waves): the segment count is the same for every sequence, half of a mixed batch's workgroups are
+  // token groups without tokens, and segments of a chunk or two cost more to start and to merge than to stream. 24
+  // decodes over 600 to 14500 keys beside a chunk (24 q / 4 KV heads of 256, int8 keys): 183 against 197 us. Batches of
+  // short sequences alone are better without: their small segments fill the launch's tail (32 sequences over 2100 to
+  // 65000 keys: 181 us, 185 with the floor; 64 over 270 to 7400 keys of 8 heads of 128: 70 and 73 us).
+  P.min_keys = P.routed && 4 * (int64_t)a->num_seqs * cache->num_kv_heads >= device_cus() ? 512 : 0;
   if (P.segm_rows > 0) {  // no more segments than keep the device's CUs busy, as the workspace grows with them
     const int64_t pairs = (int64_t)a->num_seqs * cache->num_kv_heads;
     const int64_t want = (8 * (int64_t)device_cus() + pairs - 1) / pairs;
@@ -229,10 +237,10 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
     // rows above the cap (or two row tiles at head 512) run as token groups on the tokens' own rows
     const int rows = a->max_query_len * G;
     const bool groups = rows > max_rows || (rows > 16 && cache->head_size == 512);
-    int st = groups ? decode_routed(cache, &P.decode, nullptr, max_rows, s) : qp_decode_splitkv(cache, &P.decode, stream);
+    int st = groups ? decode_routed(cache, &P.decode, nullptr, max_rows, P.min_keys, s) : decode_plain(cache, &P.decode, P.min_keys, s);
     if (st != QP_OK) return st;
     const qp_merge_args m = merge_of(P.decode, a, cache->head_size);
-    return qp_merge_segments(&m, stream);
+    return merge_routed(&m, nullptr, nullptr, 0, nullptr, P.min_keys, s);
   }
   P.prefill.workspace = P.prefill.workspace_bytes > 0 ? ws + P.off_prefill : nullptr;
   if (!P.routed) return prefill_run(cache, &P.prefill, nullptr, s);
@@ -247,10 +255,10 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
   if (st != QP_OK) return st;
   // mixed batches: groups of at most 16 rows (one row tile) whatever max_decode_rows says, as the host does not know
   // each short sequence's query count here
-  st = decode_routed(cache, &P.decode, route_row, 16, s);
+  st = decode_routed(cache, &P.decode, route_row, 16, P.min_keys, s);
   if (st != QP_OK) return st;
   const qp_merge_args m = merge_of(P.decode, a, cache->head_size);
-  return merge_routed(&m, row_tok, row_seq, P.rows_cap, nullptr, 0, s);
+  return merge_routed(&m, row_tok, row_seq, P.rows_cap, nullptr, P.min_keys, s);
 }
 
 // ------------------------------------------------------------------------------ entry point without allocation

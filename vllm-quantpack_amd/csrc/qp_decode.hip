@@ -1642,6 +1642,7 @@ int check_merge(const qp_merge_args *a) {
 }
 
 constexpr int kWaveMergeSegments = 16;  // merges of at most this many segments run one wave per row
+constexpr int kWaveMergeRows = 1024;    // and so do merges of this many rows, where segments have a floor
 
 template <int CPL>
 void launch_merge_wave(const MergeParams &p, dim3 grid, int rows, hipStream_t s) {
@@ -1654,7 +1655,8 @@ void launch_merge_wave(const MergeParams &p, dim3 grid, int rows, hipStream_t s)
 int launch_merge(const MergeParams &p, int64_t rows, int num_q_heads, hipStream_t s) {
   if (rows <= 0) return QP_OK;
   const bool pow2 = (p.head_size & (p.head_size - 1)) == 0;
-  if (p.num_segments <= kWaveMergeSegments && p.head_size >= 64 && pow2 && rows <= INT32_MAX) {
+  const bool many = p.min_keys > 0 && rows * num_q_heads >= kWaveMergeRows;
+  if ((p.num_segments <= kWaveMergeSegments || many) && p.head_size >= 64 && pow2 && rows <= INT32_MAX) {
     // few segments: one wave per row (a workgroup per row would leave most of its threads idle)
     const dim3 grid((unsigned)((rows + 3) / 4), num_q_heads);
     const int r = (int)rows;
@@ -1677,7 +1679,10 @@ int launch_merge(const MergeParams &p, int64_t rows, int num_q_heads, hipStream_
 
 }  // namespace
 
-extern "C" int qp_decode_splitkv(const qp_paged_cache *cache, const qp_decode_args *a, qp_stream_t stream) {
+namespace qp {
+
+// Split-KV decode of a batch of short sequences whose rows are the tokens' own.
+int decode_plain(const qp_paged_cache *cache, const qp_decode_args *a, int min_keys, hipStream_t s) {
   const int st = check_decode(cache, a, false);
   if (st != QP_OK) return st;
   if (a->num_seqs == 0 || a->num_tokens == 0) return QP_OK;
@@ -1685,6 +1690,7 @@ extern "C" int qp_decode_splitkv(const qp_paged_cache *cache, const qp_decode_ar
   const int rows = a->max_query_len * G;
   DecodeParams p;
   decode_params(cache, a, p);
+  p.min_keys = min_keys;
   int nct = rows > 16 ? 2 : 1;
   if (nct == 2 && cache->head_size == 512) {
     // Two row tiles at head 512 do not fit the registers (the accumulators alone fill the AGPRs); workgroups of
@@ -1694,7 +1700,13 @@ extern "C" int qp_decode_splitkv(const qp_paged_cache *cache, const qp_decode_ar
     nct = 1;
   }
   const dim3 grid(a->num_segments, cache->num_kv_heads, a->num_seqs * p.tok_groups);
-  return dispatch_hs(cache, p, nct, grid, reinterpret_cast<hipStream_t>(stream));
+  return dispatch_hs(cache, p, nct, grid, s);
+}
+
+}  // namespace qp
+
+extern "C" int qp_decode_splitkv(const qp_paged_cache *cache, const qp_decode_args *a, qp_stream_t stream) {
+  return decode_plain(cache, a, 0, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int qp_merge_segments(const qp_merge_args *a, qp_stream_t stream) {
@@ -1711,7 +1723,7 @@ namespace qp {
 // query count of each sequence need not be known on the host. With route_row, sequence i's query tokens take the
 // segment-buffer rows route_row[i] .. + T_i - 1 (route_row[i] < 0: served elsewhere); without it, their own indices.
 int decode_routed(const qp_paged_cache *cache, const qp_decode_args *a, const int32_t *route_row, int max_rows,
-                  hipStream_t s) {
+                  int min_keys, hipStream_t s) {
   const int st = check_decode(cache, a, route_row != nullptr);
   if (st != QP_OK) return st;
   if (a->num_seqs == 0 || a->num_tokens == 0) return QP_OK;
@@ -1719,6 +1731,7 @@ int decode_routed(const qp_paged_cache *cache, const qp_decode_args *a, const in
   DecodeParams p;
   decode_params(cache, a, p);
   p.route_row = route_row;
+  p.min_keys = min_keys;
   int nct = 1;
   if (G <= 16) {
     int cap = max_rows > 16 && cache->head_size != 512 ? 32 : 16;  // two row tiles or one
