@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <string>
+#include <type_traits>
 
 #include "quantpack.h"
 
@@ -245,6 +246,61 @@ __device__ __forceinline__ void fwht_lanes(float (&x)[CPL], int lane) {
       x[i] = upper ? other - x[i] : x[i] + other;
     }
   }
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+
+// The butterfly of the Walsh-Hadamard transform over lane bit M: the lower lane gets lower + upper, the upper one lower -
+// upper. sign: -1 in upper lanes, +1 in lower ones (the product is exact, so the fma rounds once, as the sum does).
+template <int M>
+__device__ __forceinline__ float lane_butterfly(float x, float sign) {
+  if constexpr (M == 1) {
+    return fmaf(x, sign, dpp<0xB1>(x));  // quad_perm (1, 0, 3, 2)
+  } else if constexpr (M == 2) {
+    return fmaf(x, sign, dpp<0x4E>(x));  // quad_perm (2, 3, 0, 1)
+  } else if constexpr (M == 4) {
+    return fmaf(x, sign, dpp<0x1B>(dpp<0x141>(x)));  // row_half_mirror (l ^ 7), then quad_perm (3, 2, 1, 0) (l ^ 3)
+  } else if constexpr (M == 8) {
+    return fmaf(x, sign, dpp<0x128>(x));  // row_ror 8
+  } else {  // a row (half) swap gives both lanes of a pair the lower and the upper value
+    const uint32_t b = __float_as_uint(x);
+    const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(b, b, false, false)
+                           : __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return fmaf(__uint_as_float(r[1]), sign, __uint_as_float(r[0]));
+  }
+}
+
+// The Walsh-Hadamard transform of rows held by groups of LANES consecutive lanes (8 to 64), E channels per lane: the
+// butterflies over channel bits in ascending order, as fwht_lanes, with every exchange on the VALU. lane: the lane's
+// number (in the wave or in its group).
+template <int E, int LANES>
+__device__ __forceinline__ void fwht_groups(float (&x)[E], int lane) {
+#pragma unroll
+  for (int span = 1; span < E; span <<= 1)
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+      if (!(i & span)) {
+        const float a = x[i], b = x[i + span];
+        x[i] = a + b;
+        x[i + span] = a - b;
+      }
+  auto stage = [&](auto tag) {
+    constexpr int M = decltype(tag)::value;
+    if constexpr (M < LANES) {
+      const float sign = (lane & M) ? -1.f : 1.f;
+#pragma unroll
+      for (int i = 0; i < E; ++i) x[i] = lane_butterfly<M>(x[i], sign);
+    }
+  };
+  stage(std::integral_constant<int, 1>{});
+  stage(std::integral_constant<int, 2>{});
+  stage(std::integral_constant<int, 4>{});
+  stage(std::integral_constant<int, 8>{});
+  stage(std::integral_constant<int, 16>{});
+  stage(std::integral_constant<int, 32>{});
 }
 
 // One query row as bf16 (E channels per lane group, 16-byte aligned rows), rotated first when signs is set. The

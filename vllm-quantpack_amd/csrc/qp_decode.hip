@@ -1063,7 +1063,7 @@ struct MergeParams {
   const float *smax, *ssum;
   int64_t sts0, sts1;
   const int32_t *cu_q, *used_k;
-  int32_t num_seqs, num_segments, head_size;
+  int32_t num_seqs, num_heads, num_segments, head_size;
   int32_t min_keys;  // floor of a segment's length (segment_keys)
   uint16_t *out;
   int64_t os0, os1;
@@ -1094,26 +1094,6 @@ __device__ __forceinline__ bool merge_row_owner(const MergeParams &p, int srow, 
   }
   seq = lo;
   return !(p.skip_seq && p.skip_seq[lo] >= 0);
-}
-
-template <int CPL>
-__device__ __forceinline__ void load_channels(const float *src, float (&v)[CPL]) {
-  if constexpr (CPL >= 4) {
-#pragma unroll
-    for (int i = 0; i < CPL / 4; ++i) {
-      const float4 x = reinterpret_cast<const float4 *>(src)[i];
-      v[4 * i] = x.x;
-      v[4 * i + 1] = x.y;
-      v[4 * i + 2] = x.z;
-      v[4 * i + 3] = x.w;
-    }
-  } else if constexpr (CPL == 2) {
-    const float2 x = *reinterpret_cast<const float2 *>(src);
-    v[0] = x.x;
-    v[1] = x.y;
-  } else {
-    v[0] = *src;
-  }
 }
 
 // One workgroup of 256 threads per (token, query head). Thread t owns channels 4 (t % (HS/4)) .. +3 of the segments
@@ -1326,47 +1306,54 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
   }
 }
 
-// One wave per (row, query head), four rows per workgroup, for merges of few segments (the key splits of a prefill
-// chunk, decode batches of many sequences at 16 segments or fewer): every lane folds every segment of its channels
-// CPL l .. CPL l + CPL - 1 (head size 64 CPL), so no state is exchanged between lanes or waves. The row's statistics
-// are wave-uniform. Segments go in batches whose loads are all issued before any is used. With signs the merged row is rotated back in registers (fwht_lanes).
-template <bool RHT, int CPL>
+// Groups of HS / 8 lanes per (row, query head), for merges of few segments (the key splits of a prefill chunk, decode
+// batches of many sequences): every lane folds every segment of its 8 channels, so no state is exchanged between lanes or
+// waves. A wave takes 512 / HS heads of one row, four rows per workgroup, so the row's token, sequence and segment count are
+// wave-uniform. Segments go in batches whose loads are all issued before any is used. With signs the merged row is
+// rotated back in registers (fwht_groups). Bound by memory latency: a wave per (row, head) with HS / 64 channels per lane had
+// 8 to 16 bytes per lane in flight and split. 512 rows x 32 heads of 64, 4 splits (19 MB): 5.5 us against 12.6 that way; 1024
+// rows x 24 heads of 256, 2 splits (63 MB): 13.0 us against 22.8; 64 decodes of 32 heads of 128: 4.7 against 4.8.
+template <bool RHT, int HS>
 __global__ __launch_bounds__(256) void merge_wave_kernel(const MergeParams p, int rows) {
+  constexpr int LANES = HS / 8;
   const int lane = threadIdx.x & 63;
   const int srow = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
-  const int head = blockIdx.y;
+  const int head = blockIdx.y * (64 / LANES) + lane / LANES;
   if (srow >= rows) return;
   int tok, seq;
   if (!merge_row_owner(p, srow, tok, seq)) return;
+  if (head >= p.num_heads) return;  // (whole lane groups)
+  const int c0 = 8 * (lane % LANES);
   const int n = p.used_k[seq];
   const int seg = segment_keys(n, p.num_segments, p.min_keys);
   const int active = seg > 0 ? min(p.num_segments, (n + seg - 1) / seg) : 0;
   const float *mrow = p.smax + (int64_t)srow * p.sts0 + (int64_t)head * p.sts1;
   const float *lrow = p.ssum + (int64_t)srow * p.sts0 + (int64_t)head * p.sts1;
-  const float *orow = p.so + (int64_t)srow * p.sos0 + (int64_t)head * p.sos1 + CPL * lane;
-  float sgn[CPL];
+  const float *orow = p.so + (int64_t)srow * p.sos0 + (int64_t)head * p.sos1 + c0;
+  float sgn[8];
   if constexpr (RHT) {
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) sgn[i] = p.signs[CPL * lane + i] * p.out_scale;
+    for (int i = 0; i < 8; ++i) sgn[i] = p.signs[c0 + i] * p.out_scale;
   }
-  constexpr int kBatch = CPL >= 4 ? 64 / CPL : 16;  // at most 64 partial floats in flight per lane
+  constexpr int kBatch = 8;
   float mt = -INFINITY, lt = 0.f;
-  float a[CPL];
+  float a[8];
 #pragma unroll
-  for (int i = 0; i < CPL; ++i) a[i] = 0.f;
+  for (int i = 0; i < 8; ++i) a[i] = 0.f;
   for (int s0 = 0; s0 < active; s0 += kBatch) {
-    float v[kBatch][CPL];
+    float4 v[kBatch][2];
     float ms[kBatch], ls[kBatch];
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) {
       const int s = s0 + k;
       if (s < active) {
-        load_channels<CPL>(orow + (int64_t)s * p.sos2, v[k]);
+        const float4 *src = reinterpret_cast<const float4 *>(orow + (int64_t)s * p.sos2);
+        v[k][0] = src[0];
+        v[k][1] = src[1];
         ms[k] = mrow[s];
         ls[k] = lrow[s];
       } else {
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) v[k][i] = 0.f;
+        v[k][0] = v[k][1] = make_float4(0.f, 0.f, 0.f, 0.f);
         ms[k] = -INFINITY;
         ls[k] = 0.f;
       }
@@ -1377,41 +1364,43 @@ __global__ __launch_bounds__(256) void merge_wave_kernel(const MergeParams p, in
     if (bm == -INFINITY) continue;
     const float f = mt == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mt - bm);
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) a[i] *= f;
+    for (int i = 0; i < 8; ++i) a[i] *= f;
     lt *= f;
     mt = bm;
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) {
       if (ms[k] == -INFINITY) continue;  // an empty segment: its row was not written
       const float wgt = __builtin_amdgcn_exp2f(ms[k] - mt);
+      const float x[8] = {v[k][0].x, v[k][0].y, v[k][0].z, v[k][0].w, v[k][1].x, v[k][1].y, v[k][1].z, v[k][1].w};
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) a[i] = fmaf(v[k][i], wgt, a[i]);
+      for (int i = 0; i < 8; ++i) a[i] = fmaf(x[i], wgt, a[i]);
       lt = fmaf(ls[k], wgt, lt);
     }
   }
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
 #pragma unroll
-  for (int i = 0; i < CPL; ++i) a[i] *= inv;
+  for (int i = 0; i < 8; ++i) a[i] *= inv;
   if constexpr (RHT) {
-    fwht_lanes<CPL>(a, lane);
+    fwht_groups<8, LANES>(a, lane);
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) a[i] *= sgn[i];
+    for (int i = 0; i < 8; ++i) a[i] *= sgn[i];
   }
-  uint16_t *dst = p.out + (int64_t)tok * p.os0 + (int64_t)head * p.os1 + CPL * lane;
-  if constexpr (CPL >= 2) {
-    if ((reinterpret_cast<uintptr_t>(p.out + (int64_t)tok * p.os0 + (int64_t)head * p.os1) & 3) == 0) {
+  uint16_t *dst = p.out + (int64_t)tok * p.os0 + (int64_t)head * p.os1 + c0;
+  u32x4_t w;
 #pragma unroll
-      for (int i = 0; i < CPL; i += 2)
-        reinterpret_cast<uint32_t *>(dst)[i / 2] =
-            (uint32_t)f32_to_bf16_bits(a[i]) | ((uint32_t)f32_to_bf16_bits(a[i + 1]) << 16);
-    } else {
+  for (int i = 0; i < 4; ++i)
+    w[i] = (uint32_t)f32_to_bf16_bits(a[2 * i]) | ((uint32_t)f32_to_bf16_bits(a[2 * i + 1]) << 16);
+  const uint32_t at = (uint32_t)reinterpret_cast<uintptr_t>(dst);
+  if ((at & 15) == 0) {
+    *reinterpret_cast<u32x4_t *>(dst) = w;
+  } else if ((at & 3) == 0) {
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) dst[i] = f32_to_bf16_bits(a[i]);
-    }
+    for (int i = 0; i < 4; ++i) reinterpret_cast<uint32_t *>(dst)[i] = w[i];
   } else {
-    dst[0] = f32_to_bf16_bits(a[0]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[i] = (uint16_t)(w[i / 2] >> (16 * (i & 1)));
   }
-  if (p.lse && lane == 0)
+  if (p.lse && lane % LANES == 0)
     p.lse[(int64_t)tok * p.ls0 + (int64_t)head * p.ls1] =
         (mt == -INFINITY || lt <= 0.f) ? -INFINITY : (mt + __log2f(lt)) * 0.6931471805599453f;
 }
@@ -1610,6 +1599,7 @@ MergeParams merge_params(const qp_merge_args *a) {
   p.cu_q = a->cu_seqlens_q;
   p.used_k = a->seqused_k;
   p.num_seqs = a->num_seqs;
+  p.num_heads = a->num_q_heads;
   p.num_segments = a->num_segments;
   p.min_keys = 0;
   p.head_size = a->head_size;
@@ -1641,33 +1631,32 @@ int check_merge(const qp_merge_args *a) {
   return QP_OK;
 }
 
-constexpr int kWaveMergeSegments = 16;  // merges of at most this many segments run one wave per row
+constexpr int kWaveMergeSegments = 16;  // merges of at most this many segments run without sharing a row
 constexpr int kWaveMergeRows = 1024;    // and so do merges of this many rows, where segments have a floor
 
-template <int CPL>
-void launch_merge_wave(const MergeParams &p, dim3 grid, int rows, hipStream_t s) {
-  if (p.signs) merge_wave_kernel<true, CPL><<<grid, 256, 0, s>>>(p, rows);
-  else merge_wave_kernel<false, CPL><<<grid, 256, 0, s>>>(p, rows);
+template <int HS>
+void launch_merge_wave(const MergeParams &p, int rows, hipStream_t s) {
+  constexpr int kHeads = 512 / HS;  // per wave
+  const dim3 grid((unsigned)((rows + 3) / 4), (p.num_heads + kHeads - 1) / kHeads);
+  if (p.signs) merge_wave_kernel<true, HS><<<grid, 256, 0, s>>>(p, rows);
+  else merge_wave_kernel<false, HS><<<grid, 256, 0, s>>>(p, rows);
 }
 
-// Per query head: one wave per row (token, or segment-buffer row when routed) for few segments, else one workgroup
-// per row.
+// Per query head: HS / 8 lanes per row (token, or segment-buffer row when routed) for few segments (a workgroup per row
+// would leave most of its threads idle: the two key splits of a 1024-token chunk merged in 78 us that way, in 22 with a
+// wave per row), else one workgroup per row. 16-byte aligned rows are checked for (check_merge).
 int launch_merge(const MergeParams &p, int64_t rows, int num_q_heads, hipStream_t s) {
   if (rows <= 0) return QP_OK;
-  const bool pow2 = (p.head_size & (p.head_size - 1)) == 0;
   const bool many = p.min_keys > 0 && rows * num_q_heads >= kWaveMergeRows;
-  if ((p.num_segments <= kWaveMergeSegments || many) && p.head_size >= 64 && pow2 && rows <= INT32_MAX) {
-    // few segments: one wave per row (a workgroup per row would leave most of its threads idle)
-    const dim3 grid((unsigned)((rows + 3) / 4), num_q_heads);
+  if ((p.num_segments <= kWaveMergeSegments || many) && rows <= INT32_MAX - 3) {
     const int r = (int)rows;
     switch (p.head_size) {
-      case 64: launch_merge_wave<1>(p, grid, r, s); break;
-      case 128: launch_merge_wave<2>(p, grid, r, s); break;
-      case 256: launch_merge_wave<4>(p, grid, r, s); break;
-      case 512: launch_merge_wave<8>(p, grid, r, s); break;
-      default: launch_merge_wave<16>(p, grid, r, s); break;
+      case 64: launch_merge_wave<64>(p, r, s); return launch_status();
+      case 128: launch_merge_wave<128>(p, r, s); return launch_status();
+      case 256: launch_merge_wave<256>(p, r, s); return launch_status();
+      case 512: launch_merge_wave<512>(p, r, s); return launch_status();
+      default: break;  // (16, 32 and 1024: a workgroup per row)
     }
-    return launch_status();
   }
   // a few rows need the channel split to spread the partial reads over more CUs; many rows fill the device alone
   const int parts = (p.signs || rows * num_q_heads >= 1024 || p.head_size < 64) ? 1 : 4;

@@ -18,8 +18,6 @@
 // this takes 11.2-11.6, set by the VALU work of the rotation and the quantiser's divisions as much as by memory.
 #include "qp_common.h"
 
-#include <type_traits>
-
 namespace qp {
 
 struct StoreParams {
@@ -44,31 +42,6 @@ struct StoreParams {
 __device__ __forceinline__ float round_half_away(float x) { return x >= 0.f ? truncf(x + 0.5f) : truncf(x - 0.5f); }
 
 constexpr int kStoreThreads = 256;
-
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-
-// The butterfly of the Walsh-Hadamard transform over lane bit M: the lower lane gets lower + upper, the upper one lower -
-// upper. sign: -1 in upper lanes, +1 in lower ones (the product is exact, so the fma rounds once, as the sum does).
-template <int M>
-__device__ __forceinline__ float lane_butterfly(float x, float sign) {
-  if constexpr (M == 1) {
-    return fmaf(x, sign, dpp<0xB1>(x));  // quad_perm (1, 0, 3, 2)
-  } else if constexpr (M == 2) {
-    return fmaf(x, sign, dpp<0x4E>(x));  // quad_perm (2, 3, 0, 1)
-  } else if constexpr (M == 4) {
-    return fmaf(x, sign, dpp<0x1B>(dpp<0x141>(x)));  // row_half_mirror (l ^ 7), then quad_perm (3, 2, 1, 0) (l ^ 3)
-  } else if constexpr (M == 8) {
-    return fmaf(x, sign, dpp<0x128>(x));  // row_ror 8
-  } else {  // a row (half) swap gives both lanes of a pair the lower and the upper value
-    const uint32_t b = __float_as_uint(x);
-    const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(b, b, false, false)
-                           : __builtin_amdgcn_permlane32_swap(b, b, false, false);
-    return fmaf(__uint_as_float(r[1]), sign, __uint_as_float(r[0]));
-  }
-}
 
 // Maximum over the LANES lanes of a row, every lane receiving it (a group's lanes agree after each step, so mirrors serve
 // as exchanges).
@@ -116,29 +89,7 @@ __device__ __forceinline__ void store_row(float (&x)[8], u32x4_t v, const float 
   if constexpr (ROT) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] *= signs[i];
-#pragma unroll
-    for (int span = 1; span < 8; span <<= 1)
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (!(i & span)) {
-          const float a = x[i], b = x[i + span];
-          x[i] = a + b;
-          x[i + span] = a - b;
-        }
-    auto stage = [&](auto tag) {
-      constexpr int M = decltype(tag)::value;
-      if constexpr (M < LANES) {
-        const float sign = (lane & M) ? -1.f : 1.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = lane_butterfly<M>(x[i], sign);
-      }
-    };
-    stage(std::integral_constant<int, 1>{});
-    stage(std::integral_constant<int, 2>{});
-    stage(std::integral_constant<int, 4>{});
-    stage(std::integral_constant<int, 8>{});
-    stage(std::integral_constant<int, 16>{});
-    stage(std::integral_constant<int, 32>{});
+    fwht_groups<8, LANES>(x, lane);
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = __uint_as_float((uint32_t)f32_to_bf16_bits(x[i]) << 16);
   }
