@@ -9,6 +9,7 @@
 //     buffers, or of the workspace when the batch can have more such rows than the buffers; the decode kernel serves
 //     them in token groups and the merge writes their output;
 //   * every other sequence takes the MFMA prefill kernel (or its query-slice path), which skips the short ones.
+// One longer sequence alone goes to the prefill kernel without a table.
 // A batch with short sequences only keeps the tokens' own rows and no table, so it needs no workspace and can be
 // recorded in a HIP graph. The randomized Hadamard rotation is fused: the kernels rotate each query row as it loads
 // and the merge / the prefill epilogue rotate the output back before the one bf16 store.
@@ -130,7 +131,12 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
       segm && (hs == 64 || hs == 128 || hs == 256 || hs == 512) && G >= 1 && G <= 32 && (hs != 512 || G <= 16);
   P.plain_decode = decode_shape && a->max_query_len >= 1 && a->max_query_len <= QP_DECODE_MAX_QUERY &&
                    a->max_query_len * G <= 32;
-  P.routed = decode_shape && !P.plain_decode;
+  // A single sequence of more than QP_DECODE_MAX_QUERY tokens needs no table to go to the prefill kernel: the route kernel
+  // and the decode and merge launches that find nothing to do took 10 us of 55 (512 tokens of 32 heads of 64 over 4096).
+  const bool one_chunk =
+      a->num_seqs == 1 && a->num_tokens > QP_DECODE_MAX_QUERY && a->max_query_len > QP_DECODE_MAX_QUERY;
+  const bool tables = decode_shape && !P.plain_decode;  // the workspace has the sequences' table, used or not
+  P.routed = tables && !one_chunk;
   // Rows of partials the batch's short sequences can have. The caller's segment buffers hold them when they have that
   // many rows; otherwise the partials go to the workspace, so every short sequence takes the split-KV kernel (an
   // engine that allocates 128 / KV heads rows sends larger batches than that: 64 sequences over up to 8192 keys at 32
@@ -138,7 +144,7 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
   const int64_t cap = (int64_t)QP_DECODE_MAX_QUERY * a->num_seqs;
   const int64_t rows = a->num_tokens < cap ? a->num_tokens : cap;
   P.rows_cap = P.routed ? (int)rows : 0;
-  P.segm_rows = decode_shape && rows > a->segm_rows ? rows : 0;
+  P.segm_rows = (P.plain_decode || P.routed) && rows > a->segm_rows ? rows : 0;
 
   qp_decode_args &d = P.decode;
   d.query = a->query;
@@ -199,7 +205,7 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
 
   // workspace: [route_row | row_tok | row_seq | split-KV partials | prefill workspace]
   P.off_route = 0;
-  P.off_tok = P.routed ? up256(4 * (int64_t)a->num_seqs) : 0;
+  P.off_tok = tables ? up256(4 * (int64_t)a->num_seqs) : 0;
   P.off_seq = P.off_tok + (P.routed ? up256(4 * (int64_t)P.rows_cap) : 0);
   P.off_segm = P.off_seq + (P.routed ? up256(4 * (int64_t)P.rows_cap) : 0);
   P.off_prefill =
