@@ -65,7 +65,7 @@ int qp_unpack_segment(const qp_cache_half *half, int32_t block_size, int32_t num
                       const int64_t out_stride[2], qp_stream_t stream);
 
 /*
- * Split-KV decode over a paged int4 / k8v4 cache (head 128, 256 or 512) for batches whose sequences have
+ * Split-KV decode over a paged int4 / k8v4 cache (head 64, 128, 256 or 512) for batches whose sequences have
  * 1..QP_DECODE_MAX_QUERY query tokens: one workgroup per (segment, KV head, sequence) holds every query row of the KV head's GQA group, so the
  * cache is read once per step. Writes unnormalised fp32 segment partials; qp_merge_segments finishes.
  * Replaces the generated _launch_packed_attn_qp / _launch_k8v4_qp 3D path and _attn_packed_qp / _attn_k8v4_qp
@@ -134,11 +134,10 @@ int qp_merge_segments(const qp_merge_args *args, qp_stream_t stream);
  * When the query blocks alone cannot fill the device, the keys of each block are split over workgroups
  * (num_splits, 0 = chosen for the device) whose fp32 partials go to the caller's workspace and are merged as in
  * qp_merge_segments; without enough workspace an automatic choice falls back to one split.
- * Rows are (token, query head) pairs, so any GQA width fills the MFMA tiles. Head 128 from 8 query heads per KV head
- * runs a wide variant on 32-row MFMA tiles; head 512 with int4 keys runs that variant too, always with at least 2
- * splits; with int8 keys, and head 64, it runs the
- * split-KV decode kernel over causal query slices of at most 4 tokens and merges. These paths need the workspace
- * (qp_prefill_workspace_size bytes, 256-byte aligned).
+ * Rows are (token, query head) pairs, so any GQA width (at head 64, up to 32 query heads per KV head) fills the MFMA
+ * tiles. Head 512 with int4 keys always runs with at least 2 splits; with int8 keys it runs the split-KV decode kernel
+ * over causal query slices of at most 4 tokens and merges. Head 512 needs the workspace (qp_prefill_workspace_size
+ * bytes, 256-byte aligned).
  * With rht_signs the result is rotated back, out = (o H D) * rht_out_scale, as qp_merge_segments does.
  * Replaces prefill_sequence (int4_prefill.py:203-232: unpack to bf16 segments + FlashAttention + LSE merge, with the
  * inverse single_rht of int4_kv.py:329) and the 2D path of the generated Triton kernel (int4_kv.py:113-118).
@@ -159,7 +158,7 @@ typedef struct qp_prefill_args {
   float softmax_scale;
   void *out;                   /* bf16 [num_tokens, num_q_heads, head_size] */
   int64_t out_stride[2];
-  void *workspace;             /* >= qp_prefill_workspace_size bytes, 256-byte aligned; may be NULL for head 128 / 256 */
+  void *workspace;             /* >= qp_prefill_workspace_size bytes, 256-byte aligned; may be NULL below head 512 */
   int64_t workspace_bytes;
   const float *rht_signs;      /* optional: inverse rotation of the output (needs a contiguous out) */
   float rht_out_scale;

@@ -1,4 +1,4 @@
-// Pieces shared by the prefill kernels (qp_prefill.hip, qp_prefill_wide.hip): launch parameters, tile shapes of the
+// Pieces shared by the prefill kernels (qp_prefill.hip, qp_prefill_dual.hip, qp_prefill_wide.hip): launch parameters, tile shapes of the
 // packed cells, the HBM -> LDS copy plan of a tile's page runs and its block-table walk.
 #pragma once
 

@@ -895,6 +895,12 @@ void dispatch_nt(const PrefillParams &p, int nt, dim3 grid, bool span, hipStream
   else launch_prefill<HS, KFMT, 3>(p, grid, span, s);
 }
 
+// Keys of a split at least, where the split count is the host's choice: the host knows the batch's longest context only,
+// and shorter sequences need not be cut into as many splits. A 509-token chunk over 2557 keys (24 q / 4 KV heads of 256,
+// int8 keys) beside decodes over up to 16384 was cut into 7 splits of 384 keys, with 90 MB of partials: 130 us and 20 us
+// of merge; with 3 splits 84 and 14 us.
+constexpr int kMinSplitKeys = 1024;
+
 // Which kernel serves a prefill:
 //   * heads 64 and 128: the dual kernel (qp_prefill_dual.hip), two waves per SIMD, at every GQA width and chunk length.
 //     2048 tokens over 16384 keys with 64 q / 8 KV heads of 128: 1.22-1.31 ms against 1.96 on the wide kernel's 32x32x16
@@ -908,12 +914,6 @@ void dispatch_nt(const PrefillParams &p, int nt, dim3 grid, bool span, hipStream
 //   * head 512 with int4 keys: the wide kernel (qp_prefill_wide.hip, 32x32x16 MFMAs);
 //   * head 512 with int8 keys, whose 776-byte cells do not fit the wide kernel's LDS plan: query slices of the
 //     split-KV kernel.
-// Keys of a split at least, where the split count is the host's choice: the host knows the batch's longest context only,
-// and shorter sequences need not be cut into as many splits. A 509-token chunk over 2557 keys (24 q / 4 KV heads of 256,
-// int8 keys) beside decodes over up to 16384 was cut into 7 splits of 384 keys, with 90 MB of partials: 130 us and 20 us
-// of merge; with 3 splits 84 and 14 us.
-constexpr int kMinSplitKeys = 1024;
-
 enum class PrefillPath { kSlices, kTiles, kWide, kDual };
 
 PrefillPath prefill_path(const qp_paged_cache *cache, const qp_prefill_args *a) {
@@ -1040,6 +1040,7 @@ int prefill_run(const qp_paged_cache *cache, const qp_prefill_args *a, const int
   QP_REQUIRE(cache->num_kv_heads > 0 && a->num_q_heads > 0 && a->num_q_heads % cache->num_kv_heads == 0,
              "qp_prefill: query heads must be a multiple of KV heads");
   const int G = a->num_q_heads / cache->num_kv_heads;
+  QP_SUPPORTED(hs != 64 || G <= 32, "qp_prefill: at most 32 query heads per KV head");
   QP_SUPPORTED(cache->block_size >= 16 && cache->block_size % 16 == 0,
                "qp_prefill: block size must be a multiple of 16");
   QP_REQUIRE(a->num_seqs >= 0 && a->num_tokens >= 0 && a->max_query_len >= 0 && a->max_seqlen_k >= 0,
