@@ -561,7 +561,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
 
   // ---- epilogue: zero-point sum and l from the zero-point tile (rows 0..2: lane half 0), store
   const float csum = __shfl(acc[kCt][0], col, 64);
-  const float l = __shfl(acc[kCt][1] + acc[kCt][2], col, 64);
+  float l = __shfl(acc[kCt][1] + acc[kCt][2], col, 64);
   if (!active) return;
   float x[HS / 2];  // channel 16 k + 8 h + i at x[8 k + i]
 #pragma unroll
@@ -590,6 +590,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
           u32x2_t{pack_bf16x2(x[i], x[i + 1]), pack_bf16x2(x[i + 2], x[i + 3])};
   } else {
     if (!valid) return;
+    pf_normalise_partial(m, l, x);
     float *orow = p.so + (int64_t)(q0 + tok) * p.sos0 + head * p.sos1 + (int64_t)split * HS + 8 * h;
 #pragma unroll
     for (int i = 0; i < HS / 2; i += 4)
