@@ -15,6 +15,7 @@
 // and the merge / the prefill epilogue rotate the output back before the one bf16 store.
 #include "qp_common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace qp {
@@ -129,20 +130,23 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
   const bool segm = a->segm_output && a->segm_max && a->segm_expsum && a->segm_rows > 0 && a->num_segments >= 1;
   const bool decode_shape =
       segm && (hs == 64 || hs == 128 || hs == 256 || hs == 512) && G >= 1 && G <= 32 && (hs != 512 || G <= 16);
+  // Rows of partials that the batch's short sequences can have: q may have more rows than cu_seqlens_q covers (a padded
+  // batch). On the tokens' own rows every row of q needs one, so a batch whose q has more than the segment buffers hold
+  // and than its sequences can have is routed, which numbers the covered rows only.
+  const int64_t cap = (int64_t)QP_DECODE_MAX_QUERY * a->num_seqs;
+  const int64_t rows = a->num_tokens < cap ? a->num_tokens : cap;
   P.plain_decode = decode_shape && a->max_query_len >= 1 && a->max_query_len <= QP_DECODE_MAX_QUERY &&
-                   a->max_query_len * G <= 32;
+                   a->max_query_len * G <= 32 && a->num_tokens <= std::max<int64_t>(a->segm_rows, cap);
   // A single sequence of more than QP_DECODE_MAX_QUERY tokens needs no table to go to the prefill kernel: the route kernel
   // and the decode and merge launches that find nothing to do took 10 us of 55 (512 tokens of 32 heads of 64 over 4096).
   const bool one_chunk =
       a->num_seqs == 1 && a->num_tokens > QP_DECODE_MAX_QUERY && a->max_query_len > QP_DECODE_MAX_QUERY;
   const bool tables = decode_shape && !P.plain_decode;  // the workspace has the sequences' table, used or not
   P.routed = tables && !one_chunk;
-  // Rows of partials the batch's short sequences can have. The caller's segment buffers hold them when they have that
-  // many rows; otherwise the partials go to the workspace, so every short sequence takes the split-KV kernel (an
-  // engine that allocates 128 / KV heads rows sends larger batches than that: 64 sequences over up to 8192 keys at 32
-  // q / 8 KV heads took 280 us with the 48 past the buffers' 16 rows on the prefill kernel, 76 us here).
-  const int64_t cap = (int64_t)QP_DECODE_MAX_QUERY * a->num_seqs;
-  const int64_t rows = a->num_tokens < cap ? a->num_tokens : cap;
+  // The caller's segment buffers hold those partials when they have that many rows; otherwise the partials go to the
+  // workspace, so every short sequence takes the split-KV kernel (an engine that allocates 128 / KV heads rows sends
+  // larger batches than that: 64 sequences over up to 8192 keys at 32 q / 8 KV heads took 280 us with the 48 past the
+  // buffers' 16 rows on the prefill kernel, 76 us here).
   P.rows_cap = P.routed ? (int)rows : 0;
   P.segm_rows = (P.plain_decode || P.routed) && rows > a->segm_rows ? rows : 0;
 
