@@ -33,6 +33,25 @@ def test_rows_past_the_sequences(device, seqs, rows, buffers, fmt, hs, nq, nkv):
         assert O.relerr(got[sl], ref[sl]) < 5e-3, (i, O.relerr(got[sl], ref[sl]))
 
 
+@pytest.mark.parametrize("segments", [16, 64])  # (a merge of few segments, and of many)
+@pytest.mark.parametrize("rows,buffers", [(9, 3), (20, 8), (33, 3)])
+def test_output_of_rows_past_the_sequences(device, rows, buffers, segments):
+    """Where the partials go to the workspace, rows of q that no sequence covers have none: their output is left alone."""
+    import torch
+    shapes = [(2, 700), (1, 1), (2, 1300), (1, 33), (2, 64)]
+    views, table, q, cu, lens, qlens, ref = _batch(device, shapes, "int4", 650, nkv=2, hs=128, nq=8)
+    covered = q.shape[0]
+    padded = torch.ones((rows, 8, 128), dtype=torch.bfloat16, device=device)
+    padded[:covered] = q
+    out = torch.full_like(padded, -3.0)
+    segm = _segm(device, buffers, segments, nq=8, hs=128)
+    _call(views, padded, out, i32(cu, device), i32(lens, device), i32(table, device), max(qlens), max(lens), segm,
+          segments, hs=128)
+    torch.cuda.synchronize()
+    assert O.relerr(to_f32(out)[:covered], ref) < 5e-3
+    assert (out[covered:] == -3.0).all()
+
+
 def test_plan_refuses_rows_past_the_buffers(device):
     """A prepared decode step on the tokens' own rows needs a buffer row for each: refused when it is made."""
     import torch

@@ -250,7 +250,8 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
     int st = groups ? decode_routed(cache, &P.decode, nullptr, max_rows, P.min_keys, s) : decode_plain(cache, &P.decode, P.min_keys, s);
     if (st != QP_OK) return st;
     const qp_merge_args m = merge_of(P.decode, a, cache->head_size);
-    return merge_routed(&m, nullptr, nullptr, 0, nullptr, P.min_keys, s);
+    // (rows of a padded q that no sequence covers have no partials in the workspace, and their output stays as it is)
+    return merge_routed(&m, nullptr, nullptr, 0, nullptr, P.segm_rows > 0, P.min_keys, s);
   }
   P.prefill.workspace = P.prefill.workspace_bytes > 0 ? ws + P.off_prefill : nullptr;
   if (!P.routed) return prefill_run(cache, &P.prefill, nullptr, s);
@@ -268,7 +269,7 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
   st = decode_routed(cache, &P.decode, route_row, 16, P.min_keys, s);
   if (st != QP_OK) return st;
   const qp_merge_args m = merge_of(P.decode, a, cache->head_size);
-  return merge_routed(&m, row_tok, row_seq, P.rows_cap, nullptr, P.min_keys, s);
+  return merge_routed(&m, row_tok, row_seq, P.rows_cap, nullptr, false, P.min_keys, s);
 }
 
 // ------------------------------------------------------------------------------ entry point without allocation

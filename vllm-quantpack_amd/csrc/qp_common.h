@@ -124,7 +124,7 @@ int decode_plain(const qp_paged_cache *cache, const qp_decode_args *a, int min_k
 int decode_routed(const qp_paged_cache *cache, const qp_decode_args *a, const int32_t *route_row, int max_rows,
                   int min_keys, hipStream_t s);
 int merge_routed(const qp_merge_args *a, const int32_t *row_tok, const int32_t *row_seq, int64_t rows,
-                 const int32_t *skip_seq, int min_keys, hipStream_t s);
+                 const int32_t *skip_seq, bool covered_only, int min_keys, hipStream_t s);
 int prefill_run(const qp_paged_cache *cache, const qp_prefill_args *a, const int32_t *skip_seq, hipStream_t s);
 
 // Exact magic division for 0 <= x < 2^31 by d >= 2: m = ceil(2^(31+l) / d), l = ceil(log2 d);

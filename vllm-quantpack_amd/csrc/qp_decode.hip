@@ -1074,8 +1074,10 @@ struct MergeParams {
   // Routed rows: workgroup x merges segment-buffer row x for token row_tok[x] of sequence row_seq[x] (-1: unused
   // row). Without them, row x is token x.
   const int32_t *row_tok, *row_seq;
-  // Plain rows only: sequences with skip_seq[i] >= 0 are merged elsewhere (null: none).
+  // Plain rows only: sequences with skip_seq[i] >= 0 are merged elsewhere (null: none), and with covered_only the rows of
+  // q past the last sequence are left alone.
   const int32_t *skip_seq;
+  bool covered_only;
 };
 
 // The token and sequence of merge row srow (wave-uniform): false when the row is served elsewhere.
@@ -1086,6 +1088,7 @@ __device__ __forceinline__ bool merge_row_owner(const MergeParams &p, int srow, 
     return tok >= 0;
   }
   tok = srow;
+  if (p.covered_only && tok >= p.cu_q[p.num_seqs]) return false;
   int lo = 0, hi = p.num_seqs - 1;
   while (lo < hi) {  // last sequence whose first query token is <= tok
     const int mid = (lo + hi + 1) >> 1;
@@ -1114,6 +1117,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     if (tok < 0) return;
     lo = p.row_seq[srow];
   } else {
+    if (p.covered_only && tok >= p.cu_q[p.num_seqs]) return;
     int hi = p.num_seqs - 1;
     while (lo < hi) {  // last sequence whose first query token is <= tok
       const int mid = (lo + hi + 1) >> 1;
@@ -1614,6 +1618,7 @@ MergeParams merge_params(const qp_merge_args *a) {
   p.row_tok = nullptr;
   p.row_seq = nullptr;
   p.skip_seq = nullptr;
+  p.covered_only = false;
   return p;
 }
 
@@ -1737,9 +1742,9 @@ int decode_routed(const qp_paged_cache *cache, const qp_decode_args *a, const in
 
 // Merge of routed rows: segment-buffer row r (< rows) belongs to token row_tok[r] of sequence row_seq[r]
 // (row_tok[r] < 0: unused). With skip_seq and no row maps, a plain merge over the tokens leaves the sequences with
-// skip_seq[i] >= 0 alone.
+// skip_seq[i] >= 0 alone, and with covered_only the rows past the last sequence's.
 int merge_routed(const qp_merge_args *a, const int32_t *row_tok, const int32_t *row_seq, int64_t rows,
-                 const int32_t *skip_seq, int min_keys, hipStream_t s) {
+                 const int32_t *skip_seq, bool covered_only, int min_keys, hipStream_t s) {
   const int st = check_merge(a);
   if (st != QP_OK) return st;
   MergeParams p = merge_params(a);
@@ -1747,6 +1752,7 @@ int merge_routed(const qp_merge_args *a, const int32_t *row_tok, const int32_t *
   p.row_tok = row_tok;
   p.row_seq = row_seq;
   p.skip_seq = skip_seq;
+  p.covered_only = covered_only;
   return launch_merge(p, row_tok ? rows : a->num_tokens, a->num_q_heads, s);
 }
 
@@ -1870,7 +1876,7 @@ int slice_prefill(const qp_paged_cache *cache, const qp_prefill_args *a, const i
   m.out_stride[1] = a->out_stride[1];
   m.rht_signs = a->rht_signs;
   m.rht_out_scale = a->rht_out_scale;
-  return merge_routed(&m, nullptr, nullptr, 0, skip_seq, 0, s);
+  return merge_routed(&m, nullptr, nullptr, 0, skip_seq, false, 0, s);
 }
 
 }  // namespace qp

@@ -1025,7 +1025,7 @@ int prefill_merge(const PrefillParams &p, const qp_prefill_args *a, int hs, cons
   m.out_stride[1] = a->out_stride[1];
   m.rht_signs = a->rht_signs;
   m.rht_out_scale = a->rht_out_scale;
-  return merge_routed(&m, nullptr, nullptr, 0, skip_seq, p.min_keys, s);
+  return merge_routed(&m, nullptr, nullptr, 0, skip_seq, false, p.min_keys, s);
 }
 
 int prefill_run(const qp_paged_cache *cache, const qp_prefill_args *a, const int32_t *skip_seq, hipStream_t s) {
