@@ -2,8 +2,9 @@
 //
 // Reference semantics: as prefill_kernel (qp_prefill.hip), whose arithmetic this kernel keeps: bf16 query and
 // exact-integer code operands, fp32 accumulation, S = (q . (128 + k) - sum(q) (128 + zp_k)) s_k scale (int8 keys:
-// 128 sum(q)), P_v16 = bf16(P s_v) feeding the PV product and the zero-point sum (int4_kv.py:90-94), l = sum of
-// P_v16 / s_v, causal within each sequence's query chunk (replacing int4_prefill.py:203-232).
+// 128 sum(q)), P_v16 = bf16(P s_v) feeding the PV product and the zero-point sum (int4_kv.py:90-94), l in fp32 from the
+// unrounded P (at head 128 below 8 query heads per KV head: the sum of P_v16 / s_v, FOLD below), causal within each
+// sequence's query chunk (replacing int4_prefill.py:203-232).
 //
 // MI355X design. At these head sizes 32 rows' O^T accumulators, zero-point tile included, take at most 80 registers, so
 // a wave fits 256 and two waves fit a SIMD: one wave's softmax and unpack run beside the other's MFMAs. A workgroup of
@@ -60,9 +61,10 @@ struct DualShape {
   static constexpr int kKd = kKeys * kKdRow;
   static constexpr int kVs = HS * 64;                // V^T rows of a sub-tile (32 keys, four units)
   static constexpr int kVt = kSubs * kVs;
-  // per-key scalars: a, e, b (fp32 [kKeys] each), then per sub-tile four bf16 rows of 32 keys in V^T key order: 16 +
-  // zp_v, the two halves of 1 / s_v, and one that nothing fills (rows 0..2 of the zero-point tile's A operand; the
-  // results of its other rows are not used)
+  // per-key scalars: a, e, s_v (FOLD: b; fp32 [kKeys] each), then per sub-tile four bf16 rows of 32 keys in V^T key order.
+  // Row 0, 16 + zp_v, is every row of the zero-point tile's A operand, so that every lane gets its query row's sum. With
+  // FOLD rows 0..2 are that tile's first three, rows 1 and 2 the two halves of 1 / s_v; nothing fills row 3, and the
+  // results of the tile's other rows are not used.
   static constexpr int kSc = kKeys * 20;
   static constexpr int kSlots = 4, kKbufs = 3, kVbufs = 3, kScs = 4;
   static constexpr int kOffK = kSlots * kSlot;
@@ -130,7 +132,14 @@ __host__ __device__ __forceinline__ uint32_t dual_share(uint32_t pairs) {
   return (pairs & 7) == 0 ? 0 : (pairs & 3) == 0 ? 1 : (pairs & 1) == 0 ? 2 : 3;
 }
 
-template <int HS, int KFMT, bool SPAN>
+// FOLD: the value scales are folded into the scores (the QK accumulators start at b = log2(s_v) / a, so one exp2 gives
+// P s_v) and l comes out of the zero-point tile's MFMA, as in the head-256 tile kernel; it normalises by the rounded
+// weights, and a key whose value scale is 0 drops out of it. Otherwise l is summed in fp32 from the unrounded P, two VALU
+// instructions more per score. Each shape keeps the form that it has always had (dual_folds): 8 prompts of up to 2048
+// tokens, 32 q / 8 KV heads of 128: 155 us and 2.7e-3 off the 64-bit result folded, 160 us and 3.0e-3 otherwise; 2048
+// tokens over 16384 keys, 64 q / 8 KV heads: 1409 us and 3.7e-3, 1463 us and 3.8e-3; 512 tokens over 4096, 32 q / 8 KV
+// heads of 64: 48.4 us and 3.5e-3, 51.2 us and 3.6e-3.
+template <int HS, int KFMT, bool SPAN, bool FOLD>
 __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const PrefillParams p) {
   using Sh = DualShape<HS, KFMT>;
   constexpr int KT = Sh::kKeys;
@@ -189,7 +198,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
   const int tok = valid ? rr / G : 0, jh = valid ? rr % G : 0;
   const int row_pos = valid ? n - qlen + tok : kPfNoRow;  // (< 0: a context shorter than the chunk)
   bf16x8_t qop[kCs];
-  float qsum, m = -INFINITY;
+  float qsum, m = -INFINITY, l = 0.f;  // l: of the lane's keys, until the epilogue
   {
     // channels HS / 2 h .. of the row (rotated when asked, then rounded to bf16 once, as a separate rotation pass would)
     const uint16_t *src = p.q + (int64_t)(q0 + tok) * p.qs0 + (int64_t)(kvh * G + jh) * p.qs1 + HS / 2 * h;
@@ -344,17 +353,25 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
       const bool ok = tile_key(t) + kk < ke;
       const uint32_t kw = *reinterpret_cast<const uint32_t *>(pk + kk * Sh::kCell + Sh::kKeyBytes);
       const uint32_t vw = *reinterpret_cast<const uint32_t *>(pk + kk * Sh::kCell + Sh::kCell - 4);
-      float a, e, b;
-      uint16_t rhi, rlo;
-      pf_key_scalars<KFMT>(kw, vw, p.scale_log2, ok, a, e, b, rhi, rlo);
+      float a, e, x;  // x: b, or s_v
+      uint16_t rhi = 0, rlo = 0;
+      if constexpr (FOLD) {
+        pf_key_scalars<KFMT>(kw, vw, p.scale_log2, ok, a, e, x, rhi, rlo);
+      } else {
+        a = ok ? __uint_as_float(KFMT == QP_CODES_INT4 ? kw & 0xFFFFFFF0u : kw) * p.scale_log2 : 0.f;
+        e = a * (float)(128u + (kw & 0xFu));
+        x = ok ? __uint_as_float(vw & 0xFFFFFFF0u) : 0.f;
+      }
       float *kf = reinterpret_cast<float *>(sc);
       kf[kk] = a;
       if constexpr (KFMT == QP_CODES_INT4) kf[KT + kk] = e;
-      kf[2 * KT + kk] = b;
+      kf[2 * KT + kk] = x;
       uint8_t *z = sc + 12 * KT + 256 * (kk >> 5) + 16 * Sh::v_unit(kk & 31) + Sh::v_byte(kk & 31);
       *reinterpret_cast<uint16_t *>(z) = ok ? (uint16_t)(0x4180u | ((vw & 0xFu) << 3)) : 0;
-      *reinterpret_cast<uint16_t *>(z + 64) = rhi;
-      *reinterpret_cast<uint16_t *>(z + 128) = rlo;
+      if constexpr (FOLD) {
+        *reinterpret_cast<uint16_t *>(z + 64) = rhi;
+        *reinterpret_cast<uint16_t *>(z + 128) = rlo;
+      }
     };
 
     // ---- operand addresses (a swizzle depends on col alone: 32 rows are a multiple of its period)
@@ -362,7 +379,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
       return *reinterpret_cast<const bf16x8_t *>(
           kd + (32 * u + col) * Sh::kKdRow + 16 * h + 32 * cs);
     };
-    // scalar array k (0 a, 1 e, 2 b) of the lane's keys 8 q + 4 h .. of sub-tile u
+    // scalar array k (0 a, 1 e, 2 s_v or b) of the lane's keys 8 q + 4 h .. of sub-tile u
     auto scalar4 = [&](const uint8_t *sc, int k, int u, int q) {
       return *reinterpret_cast<const f32x4_t *>(sc + 4 * (k * KT + 32 * u + 8 * q + 4 * h));
     };
@@ -372,8 +389,12 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
       if constexpr (KFMT == QP_CODES_INT4) return scalar4(sc, 1, u, q);
       else return a4;
     };
-    // S^T of a sub-tile starts from the keys' biases b = log2(s_v) / a
+    // S^T of a sub-tile starts from the keys' biases b = log2(s_v) / a, or from 0
     auto start = [&](f32x16_t &s, const uint8_t *sc, int u) {
+      if constexpr (!FOLD) {
+        s = f32x16_t{};
+        return;
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const f32x4_t b = scalar4(sc, 2, u, q);
@@ -391,7 +412,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
     auto v_op = [&](int c) {
       const int ct = c % (kCt + 1), ks = c / (kCt + 1);
       return *reinterpret_cast<const bf16x8_t *>(
-          ct == kCt ? pz + 64 * (col & 3) + 16 * (2 * ks + h)
+          ct == kCt ? pz + (FOLD ? 64 * (col & 3) : 0) + 16 * (2 * ks + h)
                     : pv + 64 * (32 * ct + col) + 16 * Sh::v_swz(col, 2 * ks + h));
     };
 
@@ -424,6 +445,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
           f32x16_t sn;
           bf16x8_t kbuf[kPre], vbuf[kPre];
           float t[16];
+          f32x4_t sv4;
           u32x4_t pn[2];
 #pragma unroll
           for (int c = 0; c < kPre; ++c) {
@@ -445,8 +467,15 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
             rmax = fmaxf(fmaxf(rmax, t[4 * q]), t[4 * q + 1]);
             rmax = fmaxf(fmaxf(rmax, t[4 * q + 2]), t[4 * q + 3]);
           };
-          auto probs = [&](int i) {  // the scores carry log2(s_v): P s_v of two keys (l comes out of the PV MFMA)
-            pn[i >> 2][i & 3] = pack_bf16x2(__builtin_amdgcn_exp2f(t[2 * i]), __builtin_amdgcn_exp2f(t[2 * i + 1]));
+          auto probs = [&](int i) {  // P s_v of two keys (FOLD: the scores carry log2(s_v), and the PV MFMA sums l)
+            const float p0 = __builtin_amdgcn_exp2f(t[2 * i]), p1 = __builtin_amdgcn_exp2f(t[2 * i + 1]);
+            if constexpr (FOLD) {
+              pn[i >> 2][i & 3] = pack_bf16x2(p0, p1);
+            } else {
+              if (i % 2 == 0) sv4 = scalar4(sc, 2, u, i / 2);
+              l += p0 + p1;
+              pn[i >> 2][i & 3] = pack_bf16x2(p0 * sv4[2 * (i & 1)], p1 * sv4[2 * (i & 1) + 1]);
+            }
           };
           constexpr int kCheck = kAll / 2 - 1;  // the last step beside which scores are made
 #pragma unroll
@@ -477,8 +506,9 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
           s = sn;
           pop[0] = pn[0];
           pop[1] = pn[1];
-          // (made here: the compiler would sink the exponentials past the tile's last branch)
+          // (made here: the compiler would sink the exponentials and their sum past the tile's last branch)
           asm volatile("" : "+v"(pop[0]), "+v"(pop[1]));
+          if constexpr (!FOLD) asm volatile("" : "+v"(l));
           pv = vt + u * Sh::kVs;
           pz = sc + 12 * KT + 256 * u;
         } else {
@@ -513,6 +543,7 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
         for (int ct = 0; ct <= kCt; ++ct)
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[ct][i] = 0.f;
+        l = 0.f;
         start(s, sc_of(0), 0);
 #pragma unroll
         for (int cs = 0; cs < kCs; ++cs) s = mfma32x32x16(k_op(kd_of(0), 0, cs), qop[cs], s);
@@ -559,9 +590,14 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
     }
   }
 
-  // ---- epilogue: zero-point sum and l from the zero-point tile (rows 0..2: lane half 0), store
-  const float csum = __shfl(acc[kCt][0], col, 64);
-  float l = __shfl(acc[kCt][1] + acc[kCt][2], col, 64);
+  // ---- epilogue: the zero-point sum (FOLD: and l) from the zero-point tile (FOLD: rows 0..2, lane half 0), store
+  float csum = acc[kCt][0];
+  if constexpr (FOLD) {
+    csum = __shfl(csum, col, 64);
+    l = __shfl(acc[kCt][1] + acc[kCt][2], col, 64);
+  } else {
+    l += shfl_xor_f(l, 32);
+  }
   if (!active) return;
   float x[HS / 2];  // channel 16 k + 8 h + i at x[8 k + i]
 #pragma unroll
@@ -603,10 +639,16 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
   }
 }
 
-template <int HS, int KFMT>
+template <int HS, int KFMT, bool FOLD>
 void launch_dual(const PrefillParams &p, dim3 grid, bool span, hipStream_t s) {
-  if (span) prefill_dual_kernel<HS, KFMT, true><<<grid, kDualThreads, 0, s>>>(p);
-  else prefill_dual_kernel<HS, KFMT, false><<<grid, kDualThreads, 0, s>>>(p);
+  if (span) prefill_dual_kernel<HS, KFMT, true, FOLD><<<grid, kDualThreads, 0, s>>>(p);
+  else prefill_dual_kernel<HS, KFMT, false, FOLD><<<grid, kDualThreads, 0, s>>>(p);
+}
+
+// Whether the value scales are folded into the scores: at head 128 below 8 query heads per KV head, with a softmax scale
+// that every stored key scale (1e-6 at least) leaves well above the smallest that can be divided by.
+bool dual_folds(const PrefillParams &p, int head_size) {
+  return head_size == 128 && p.num_q_heads / p.num_kv_heads < 8 && p.scale_log2 > 1e-20f;
 }
 
 int prefill_dual_rows() { return kDualRows; }
@@ -614,12 +656,16 @@ int prefill_dual_rows() { return kDualRows; }
 void prefill_dual(const PrefillParams &p, int head_size, int key_format, dim3 grid, bool span, hipStream_t s) {
   const uint32_t share = dual_share(grid.y * grid.z);
   grid.x = ((grid.x + (1u << share) - 1) >> share) << share;
+  const bool i4 = key_format == QP_CODES_INT4;
   if (head_size == 64) {
-    if (key_format == QP_CODES_INT4) launch_dual<64, QP_CODES_INT4>(p, grid, span, s);
-    else launch_dual<64, QP_CODES_INT8>(p, grid, span, s);
+    if (i4) launch_dual<64, QP_CODES_INT4, false>(p, grid, span, s);
+    else launch_dual<64, QP_CODES_INT8, false>(p, grid, span, s);
+  } else if (dual_folds(p, head_size)) {
+    if (i4) launch_dual<128, QP_CODES_INT4, true>(p, grid, span, s);
+    else launch_dual<128, QP_CODES_INT8, true>(p, grid, span, s);
   } else {
-    if (key_format == QP_CODES_INT4) launch_dual<128, QP_CODES_INT4>(p, grid, span, s);
-    else launch_dual<128, QP_CODES_INT8>(p, grid, span, s);
+    if (i4) launch_dual<128, QP_CODES_INT4, false>(p, grid, span, s);
+    else launch_dual<128, QP_CODES_INT8, false>(p, grid, span, s);
   }
 }
 
