@@ -38,7 +38,7 @@ def _attend(device, fmt, hs, scores, T, G, splits, seed):
 
 
 @pytest.mark.parametrize("fmt,hs,G", [("int4", 64, 4), ("int8", 64, 4), ("int4", 128, 4), ("int8", 128, 4),
-                                      ("int4", 128, 8), ("int4", 256, 6)])
+                                      ("int4", 128, 8), ("int4", 256, 6), ("int4", 512, 4), ("int8", 512, 4)])
 @pytest.mark.parametrize("order", [1, -1], ids=["rising-first", "rising-last"])
 def test_splits_whose_maxima_rise_after_their_first_keys(device, fmt, hs, G, order):
     """1024 keys that start at 1 and go on at 119, and 1024 that hold one key at 128: the 992 keys at 119 weigh twice as

@@ -76,19 +76,13 @@ __device__ __forceinline__ void pf_key_scalars(uint32_t kw, uint32_t vw, float s
   e = ok ? e : 0.f;
 }
 
-// A split's partial (m, l, x: the row's reference in log2 units, its sum and its channels, both relative to 2^m) with
-// the exponent of l moved into m: the powers of two are exact, and m is then within one unit of the row's log-sum-exp.
-// The kernels whose reference stays where a split's first keys put it may have it far from the split's true maximum
-// (56 units above to 64 below it in the dual kernel); the merge weighs splits by 2^(m - max m), which is 0 from a
-// difference of 127 on, and a split could be dropped whose keys are only 2^-7 below another's.
-template <int E>
-__device__ __forceinline__ void pf_normalise_partial(float &m, float &l, float (&x)[E]) {
-  if (!(l > 0.f && l < INFINITY)) return;  // no keys (m = -inf), or a sum that is no number
-  const int k = __builtin_amdgcn_frexp_expf(l);
-  m += (float)k;
-  l = __builtin_amdgcn_ldexpf(l, -k);
-#pragma unroll
-  for (int i = 0; i < E; ++i) x[i] = __builtin_amdgcn_ldexpf(x[i], -k);
+// The exponent of a split's sum l, which the epilogues of the dual and wide kernels move into the row's reference m: they
+// store m + k, l 2^-k and the channels times 2^-k. The powers of two are exact, and m + k is within one unit of the row's
+// log-sum-exp. In those kernels m stays where a split's first keys put it and may be far from the split's true maximum (56
+// units above to 64 below it in the dual kernel, 36 and 100 in the wide one); the merge weighs splits by 2^(m - max m),
+// which is 0 from a difference of 127 on, and a split could be dropped whose keys outweigh another's.
+__device__ __forceinline__ int pf_partial_exponent(float l) {
+  return l > 0.f && l < INFINITY ? __builtin_amdgcn_frexp_expf(l) : 0;  // (no keys, or no number)
 }
 
 template <int HS, int KFMT>

@@ -626,15 +626,17 @@ __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const Prefil
           u32x2_t{pack_bf16x2(x[i], x[i + 1]), pack_bf16x2(x[i + 2], x[i + 3])};
   } else {
     if (!valid) return;
-    pf_normalise_partial(m, l, x);
+    const int k = pf_partial_exponent(l);
+#pragma unroll
+    for (int i = 0; i < HS / 2; ++i) x[i] = __builtin_amdgcn_ldexpf(x[i], -k);
     float *orow = p.so + (int64_t)(q0 + tok) * p.sos0 + head * p.sos1 + (int64_t)split * HS + 8 * h;
 #pragma unroll
     for (int i = 0; i < HS / 2; i += 4)
       *reinterpret_cast<float4 *>(orow + 16 * (i >> 3) + (i & 7)) = make_float4(x[i], x[i + 1], x[i + 2], x[i + 3]);
     if (h == 0) {
       const int64_t st = (int64_t)(q0 + tok) * p.sts0 + head * p.sts1 + split;
-      p.smax[st] = m;
-      p.ssum[st] = l;
+      p.smax[st] = m + (float)k;
+      p.ssum[st] = __builtin_amdgcn_ldexpf(l, -k);
     }
   }
 }

@@ -620,6 +620,8 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
     const int64_t head = kvh * G + (valid ? rr % G : 0);
     // (the kernel always runs split: the merge normalises and rotates the 512-channel rows)
     if (valid) {
+      const int k = pf_partial_exponent(l);
+      auto scaled = [&](float v) { return __builtin_amdgcn_ldexpf(v - csum, -k); };
       float *orow = p.so + tok * p.sos0 + head * p.sos1 + (int64_t)split * HS;
 #pragma unroll
       for (int ct = 0; ct < HS / 32; ++ct)
@@ -627,12 +629,12 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
         for (int q = 0; q < 4; ++q) {
           const f32x16_t &a = r.acc[jt][ct];
           *reinterpret_cast<float4 *>(orow + 32 * ct + 8 * q + 4 * h) =
-              make_float4(a[4 * q] - csum, a[4 * q + 1] - csum, a[4 * q + 2] - csum, a[4 * q + 3] - csum);
+              make_float4(scaled(a[4 * q]), scaled(a[4 * q + 1]), scaled(a[4 * q + 2]), scaled(a[4 * q + 3]));
         }
       if (h == 0) {
         const int64_t st = tok * p.sts0 + head * p.sts1 + split;
-        p.smax[st] = r.m[jt];
-        p.ssum[st] = l;
+        p.smax[st] = r.m[jt] + (float)k;
+        p.ssum[st] = __builtin_amdgcn_ldexpf(l, -k);
       }
     }
   }
