@@ -38,6 +38,20 @@ def test_rows_that_fit_the_segment_buffers_need_no_workspace(seqs, tokens, segm_
     assert workspace(seqs, tokens, 2, segm_rows) == 0
 
 
+@pytest.mark.parametrize("change,why", [(dict(num_segments=2049), "2048 segments"), (dict(segm_output=4100), "16-byte aligned")])
+def test_a_long_sequence_is_refused_for_its_segment_buffers(change, why):
+    """One long sequence goes to the prefill without using the segment buffers; it is refused for them all the same, as in
+    a larger batch. (The call ends there: nothing is launched on these addresses.)"""
+    from vllm_quantpack import _hip
+    lib = _hip.lib()
+    cache, args = batch(1, 64, 64, 16)
+    for name, value in change.items():
+        setattr(args, name, value)
+    args.workspace, args.workspace_bytes = 4096, lib.qp_attention_workspace_size(ctypes.byref(cache), ctypes.byref(args))
+    st = lib.qp_attention(ctypes.byref(cache), ctypes.byref(args), None)
+    assert st == _hip.QP_ERR_INVALID and why in lib.qp_last_error().decode()
+
+
 @pytest.mark.parametrize("seqs,tokens,segm_rows", [(64, 64, 16), (5, 20, 19), (4, 16, 15)])
 def test_rows_beyond_the_segment_buffers_are_kept_in_the_workspace(seqs, tokens, segm_rows):
     """The partials, [tokens, heads, segments, head size] and two statistics, and no route table beside them."""

@@ -70,6 +70,7 @@ namespace {
 struct AttentionPlan {
   bool plain_decode;  // short sequences only: decode + merge on the tokens' own rows
   bool routed;        // a route table splits the batch between decode and prefill
+  bool one_chunk;     // a single long sequence beside segment buffers: the prefill without a table
   int rows_cap;       // segment-buffer rows the route table hands out
   int64_t off_route, off_tok, off_seq, off_segm, off_prefill, total;
   int min_keys;       // floor of a segment's length
@@ -139,10 +140,10 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
                    a->max_query_len * G <= 32 && a->num_tokens <= std::max<int64_t>(a->segm_rows, cap);
   // A single sequence of more than QP_DECODE_MAX_QUERY tokens needs no table to go to the prefill kernel: the route kernel
   // and the decode and merge launches that find nothing to do took 10 us of 55 (512 tokens of 32 heads of 64 over 4096).
-  const bool one_chunk =
-      a->num_seqs == 1 && a->num_tokens > QP_DECODE_MAX_QUERY && a->max_query_len > QP_DECODE_MAX_QUERY;
   const bool tables = decode_shape && !P.plain_decode;  // the workspace has the sequences' table, used or not
-  P.routed = tables && !one_chunk;
+  P.one_chunk = tables && a->num_seqs == 1 && a->num_tokens > QP_DECODE_MAX_QUERY &&
+                a->max_query_len > QP_DECODE_MAX_QUERY;
+  P.routed = tables && !P.one_chunk;
   // The caller's segment buffers hold those partials when they have that many rows; otherwise the partials go to the
   // workspace, so every short sequence takes the split-KV kernel (an engine that allocates 128 / KV heads rows sends
   // larger batches than that: 64 sequences over up to 8192 keys at 32 q / 8 KV heads took 280 us with the 48 past the
@@ -254,7 +255,13 @@ extern "C" int qp_attention(const qp_paged_cache *cache, const qp_attention_args
     return merge_routed(&m, nullptr, nullptr, 0, nullptr, P.segm_rows > 0, P.min_keys, s);
   }
   P.prefill.workspace = P.prefill.workspace_bytes > 0 ? ws + P.off_prefill : nullptr;
-  if (!P.routed) return prefill_run(cache, &P.prefill, nullptr, s);
+  if (!P.routed) {
+    if (P.one_chunk) {  // (segment buffers that a routed batch is refused for are refused here too)
+      const int st = decode_check(cache, &P.decode);
+      if (st != QP_OK) return st;
+    }
+    return prefill_run(cache, &P.prefill, nullptr, s);
+  }
 
   int32_t *route_row = reinterpret_cast<int32_t *>(ws + P.off_route);
   int32_t *row_tok = reinterpret_cast<int32_t *>(ws + P.off_tok);

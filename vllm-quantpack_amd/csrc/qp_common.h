@@ -120,6 +120,7 @@ int slice_prefill(const qp_paged_cache *cache, const qp_prefill_args *a, const i
 // Routed split-KV decode and merge (qp_decode.hip) and prefill (qp_prefill.hip) for qp_attention: a route table
 // gives each short sequence its first segment-buffer row (route_row[i] >= 0) and sends the others to the prefill.
 // min_keys: floor of a segment's length (segment_keys), the same for a batch's decode and its merge.
+int decode_check(const qp_paged_cache *cache, const qp_decode_args *a);  // what decode_routed refuses
 int decode_plain(const qp_paged_cache *cache, const qp_decode_args *a, int min_keys, hipStream_t s);
 int decode_routed(const qp_paged_cache *cache, const qp_decode_args *a, const int32_t *route_row, int max_rows,
                   int min_keys, hipStream_t s);

@@ -1675,6 +1675,8 @@ int launch_merge(const MergeParams &p, int64_t rows, int num_q_heads, hipStream_
 
 namespace qp {
 
+int decode_check(const qp_paged_cache *cache, const qp_decode_args *a) { return check_decode(cache, a, true); }
+
 // Split-KV decode of a batch of short sequences whose rows are the tokens' own.
 int decode_plain(const qp_paged_cache *cache, const qp_decode_args *a, int min_keys, hipStream_t s) {
   const int st = check_decode(cache, a, false);
