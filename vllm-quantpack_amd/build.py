@@ -316,9 +316,16 @@ def has_inline_mfma(text):
     return re.search(r'asm\s+volatile\s*\(\s*"[^;]*?v_mfma', text) is not None
 
 
-def _check_inline_mfma(src, verbose, scheduled=False):
+def has_mfma(text):
+    """Whether a source holds an MFMA, as inline assembly or as the compiler's builtin."""
+    return has_inline_mfma(text) or "__builtin_amdgcn_mfma" in text
+
+
+def _check_mfma(src, verbose, scheduled=False):
+    """The checks of a source's generated code: the wait states around inline-assembly MFMAs, and no spill code in an MFMA
+    loop, whoever wrote its MFMAs."""
     text = open(src).read()
-    if not has_inline_mfma(text):
+    if not has_mfma(text):
         return
     out = os.path.join(OBJ, os.path.basename(src).replace(".hip", ".gfx.s"))
     if not scheduled:  # (a scheduled build wrote the assembly of the code it embedded)
@@ -340,14 +347,14 @@ def _check_inline_mfma(src, verbose, scheduled=False):
 
 def build(jobs=None, verbose=False, only=None):
     """Compile every csrc/*.hip (or only the named ones, reusing the other objects of an earlier build), check the
-    inline-MFMA wait states and link the shared library. Returns the library path."""
+    code of their MFMA loops and link the shared library. Returns the library path."""
     os.makedirs(OBJ, exist_ok=True)
     srcs = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
     todo = [s for s in srcs if not only or os.path.basename(s) in only]
     jobs = jobs or min(8, os.cpu_count() or 1, len(srcs))
     with cf.ThreadPoolExecutor(jobs) as ex:
         scheduled = dict(zip(todo, ex.map(lambda s: _compile(s, verbose), todo)))
-        list(ex.map(lambda s: _check_inline_mfma(s, verbose, scheduled[s]), todo))
+        list(ex.map(lambda s: _check_mfma(s, verbose, scheduled[s]), todo))
     objs = [os.path.join(OBJ, os.path.basename(s).replace(".hip", ".o")) for s in srcs]
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]

@@ -7,7 +7,8 @@
 // sequence's query chunk (replacing int4_prefill.py:203-232).
 //
 // MI355X design. At these head sizes 32 rows' O^T accumulators, zero-point tile included, take at most 80 registers, so
-// a wave fits 256 and two waves fit a SIMD: one wave's softmax and unpack run beside the other's MFMAs. A workgroup of
+// a wave's tile loop fits 256 (at head 128 some instances spill up to 10 around it; the build refuses spill code in it)
+// and two waves fit a SIMD: one wave's softmax and unpack run beside the other's MFMAs. A workgroup of
 // 8 waves owns 256 consecutive (token, query head) rows of one sequence and KV head (any GQA width fills them) and one
 // key split; a tile of 64 keys is unpacked once for all rows, with one barrier per tile.
 //   * 32x32x16 MFMAs: with two waves per SIMD (a loop of MFMAs with N independent FMAs after each, both waves running it)
