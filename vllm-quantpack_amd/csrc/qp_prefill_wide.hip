@@ -42,10 +42,10 @@ constexpr float kWideBias = 36.f;      // log2 units between a row's first runni
 constexpr float kWideHeadroom = 100.f; // largest score - m taken without starting the split again
 constexpr int kWidePasses = 8;         // passes over a split at most (each raises the flagged maxima by > 136)
 
-template <int HS, int KFMT>
+constexpr int HS = 512;  // with int4 keys
+using Pf = PfShape<HS, QP_CODES_INT4>;
+
 struct WShape {
-  using Pf = PfShape<HS, KFMT>;
-  static_assert(HS == 512 && KFMT == QP_CODES_INT4, "head 512 with int4 keys");
   static constexpr int kKeyBytes = Pf::kKeyBytes;
   static constexpr int kCell = Pf::kCell;
   static constexpr int kSlot = 32 * kCell;         // one packed slot (two 16-cell page runs)
@@ -76,10 +76,9 @@ __host__ __device__ constexpr int zp_pos(int kk) { return 16 * ((kk >> 2) & 1) +
 
 // The unpack of one tile's V, cut into stages that the QK phase spreads over its MFMA steps. The per-key scalars come from
 // slot pks into block sc (a tile further on).
-template <int HS, int KFMT>
 struct WStager {
-  using Sh = WShape<HS, KFMT>;
-  static constexpr int kVUnits = HS > kPfWaves * 64 ? HS / (kPfWaves * 64) : 1;  // V units per thread
+  using Sh = WShape;
+  static constexpr int kVUnits = HS / (kPfWaves * 64);  // V units per thread
   const uint8_t *pk, *pks;
   uint8_t *vt, *sc;
   int k0, kend, tid, vu;
@@ -152,20 +151,13 @@ __device__ __forceinline__ bf16x8_t k_operand(uint32_t x) {
   return as_bf16x8(u32x4_t{nib_pair(x), nib_pair(x >> 4), nib_pair(x >> 8), nib_pair(x >> 12)});
 }
 
-// Rows of the wide kernel per wave and per workgroup: NT 32-row tiles per wave.
-template <int HS>
-constexpr int wide_nt() { return 1; }  // the 32 rows' query operands take 128 VGPRs
-
-template <int HS, int NT>
+// The wave's 32 rows (their query operands take 128 VGPRs, their accumulators all AGPRs).
 struct WRows {
-  static constexpr int kCs = HS / 16;  // 16-channel QK steps
-  static constexpr int kCt = HS / 32;  // 32-channel PV tiles
-  bf16x8_t qop[NT][kCs];
-  f32x16_t acc[NT][kCt];               // O^T tiles: lane l holds row l % 32, channels 32 ct + 8 (i / 4) + 4 (l / 32) + i % 4
-  float qsum[NT], m[NT], l[NT], c[NT]; // l and c (zero-point sum) over the lane's half of each tile's keys
-  float mnext[NT];                     // the maximum to start again with (a score beyond the headroom)
-  int row_pos[NT];                     // position of the row's token (rows past the chunk: beyond every key, q = 0)
-  bool valid[NT];
+  bf16x8_t qop[HS / 16];     // 16-channel QK steps
+  f32x16_t acc[HS / 32];     // O^T tiles: lane l holds row l % 32, channels 32 ct + 8 (i / 4) + 4 (l / 32) + i % 4
+  float qsum, m, l, c;       // l and c (zero-point sum) over the lane's half of each tile's keys
+  float mnext;               // the maximum to start again with (a score beyond the headroom)
+  int row_pos;               // position of the row's token (rows past the chunk: beyond every key, q = 0)
 };
 
 // S^T += K Q^T of one 16-channel step, as inline assembly writing VGPRs. The 2 wait states before the MFMA are for a K
@@ -181,45 +173,40 @@ __device__ __forceinline__ void wqk(f32x16_t &s, bf16x8_t kop, bf16x8_t q, bool 
     asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(kop), "v"(q));
 }
 
-// Softmax of one tile for the row tiles: scores from s (S^T), per-key scalars from the tile's scalar block sc; P16 in PV operand
-// order (pop[jt][ks]). Returns true when a score exceeds its row's maximum by more than the headroom (the row's
+// Softmax of one tile: scores from s (S^T), per-key scalars from the tile's scalar block sc; P16 in PV operand order
+// (pop[ks]). Returns true when a score exceeds its row's maximum by more than the headroom (the row's
 // mnext then records the maximum to start again with; this tile's results are discarded).
-template <int HS, int KFMT, int NT, bool MASK>
-__device__ __forceinline__ bool w_softmax(WRows<HS, NT> &r, const f32x16_t (&s)[NT], const uint8_t *sc, int k0,
-                                          int kend, u32x4_t (&pop)[NT][2], int lane) {
-  using Sh = WShape<HS, KFMT>;
+template <bool MASK>
+__device__ __forceinline__ bool w_softmax(WRows &r, const f32x16_t &s, const uint8_t *sc, int k0, int kend,
+                                          u32x4_t (&pop)[2], int lane) {
+  using Sh = WShape;
   const int h = lane >> 5;
-  float t[NT][16];
+  float t[16];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const float4 a4 = *reinterpret_cast<const float4 *>(sc + Sh::kScA + 4 * (8 * q + 4 * h));
     const float4 e4 = *reinterpret_cast<const float4 *>(sc + Sh::kScE + 4 * (8 * q + 4 * h));
     const float av[4] = {a4.x, a4.y, a4.z, a4.w}, ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
-    for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float cc = fmaf(r.qsum[jt], ev[j], r.m[jt]);
-        float v = fmaf(s[jt][4 * q + j], av[j], -cc);
-        if constexpr (MASK) {
-          const int key = k0 + 8 * q + 4 * h + j;
-          if (key > r.row_pos[jt] || key >= kend) v = -INFINITY;
-        }
-        t[jt][4 * q + j] = v;
+    for (int j = 0; j < 4; ++j) {
+      const float cc = fmaf(r.qsum, ev[j], r.m);
+      float v = fmaf(s[4 * q + j], av[j], -cc);
+      if constexpr (MASK) {
+        const int key = k0 + 8 * q + 4 * h + j;
+        if (key > r.row_pos || key >= kend) v = -INFINITY;
       }
+      t[4 * q + j] = v;
+    }
   }
   bool over = false;
-#pragma unroll
-  for (int jt = 0; jt < NT; ++jt) {
-    float mx = fmaxf(fmaxf(fmaxf(t[jt][0], t[jt][1]), fmaxf(t[jt][2], t[jt][3])),
-                     fmaxf(fmaxf(t[jt][4], t[jt][5]), fmaxf(t[jt][6], t[jt][7])));
-    mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(t[jt][8], t[jt][9]), fmaxf(t[jt][10], t[jt][11])),
-                         fmaxf(fmaxf(t[jt][12], t[jt][13]), fmaxf(t[jt][14], t[jt][15]))));
-    if (__builtin_expect(__any(mx > kWideHeadroom), 0)) {
-      const float rm = fmaxf(mx, shfl_xor_f(mx, 32));  // the row's maximum over the tile (lanes l, l ^ 32)
-      if (rm > kWideHeadroom) r.mnext[jt] = fmaxf(r.mnext[jt], r.m[jt] + rm + kWideBias);
-      over = true;
-    }
+  float mx = fmaxf(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])),
+                   fmaxf(fmaxf(t[4], t[5]), fmaxf(t[6], t[7])));
+  mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(t[8], t[9]), fmaxf(t[10], t[11])),
+                       fmaxf(fmaxf(t[12], t[13]), fmaxf(t[14], t[15]))));
+  if (__builtin_expect(__any(mx > kWideHeadroom), 0)) {
+    const float rm = fmaxf(mx, shfl_xor_f(mx, 32));  // the row's maximum over the tile (lanes l, l ^ 32)
+    if (rm > kWideHeadroom) r.mnext = fmaxf(r.mnext, r.m + rm + kWideBias);
+    over = true;
   }
   const u32x4_t z0 = *reinterpret_cast<const u32x4_t *>(sc + Sh::kScZ + 32 * h);
   const u32x4_t z1 = *reinterpret_cast<const u32x4_t *>(sc + Sh::kScZ + 32 * h + 16);
@@ -229,31 +216,26 @@ __device__ __forceinline__ bool w_softmax(WRows<HS, NT> &r, const f32x16_t (&s)[
     const float4 s4 = *reinterpret_cast<const float4 *>(sc + Sh::kScS + 4 * (8 * q + 4 * h));
     const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
-    for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        const int i = 4 * q + j;
-        const float p0 = __builtin_amdgcn_exp2f(t[jt][i]);
-        const float p1 = __builtin_amdgcn_exp2f(t[jt][i + 1]);
-        r.l[jt] += p0 + p1;
-        const uint32_t pk = pack_bf16x2(p0 * sv[j], p1 * sv[j + 1]);
-        r.c[jt] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk),
-                                                  __builtin_bit_cast(bf16x2_t, zp[i / 2]), r.c[jt], false);
-        pop[jt][i / 8][(i % 8) / 2] = pk;
-      }
+    for (int j = 0; j < 4; j += 2) {
+      const int i = 4 * q + j;
+      const float p0 = __builtin_amdgcn_exp2f(t[i]);
+      const float p1 = __builtin_amdgcn_exp2f(t[i + 1]);
+      r.l += p0 + p1;
+      const uint32_t pk = pack_bf16x2(p0 * sv[j], p1 * sv[j + 1]);
+      r.c = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk), __builtin_bit_cast(bf16x2_t, zp[i / 2]),
+                                            r.c, false);
+      pop[i / 8][(i % 8) / 2] = pk;
+    }
   }
   return over;
 }
 
-// O^T += V^T P^T of one channel tile and K step for the row tiles, as inline assembly on AGPR accumulators: the
-// compiler then never moves the tiles (its own MFMAs here had all 128 accumulator registers copied at every loop
+// O^T += V^T P^T of one channel tile and K step, as inline assembly on an AGPR accumulator tile: the compiler then never
+// moves the tiles (its own MFMAs here had all 128 accumulator registers copied at every loop
 // iteration). Nothing but these MFMAs touches the tiles between the zeroing at a pass's start and the epilogue, which
 // follows wpv_drain.
-template <int NT, int CT>
-__device__ __forceinline__ void wpv_step(f32x16_t (&acc)[NT][CT], int ct, bf16x8_t vop, const u32x4_t (&p)[NT][2],
-                                         int ks) {
-  static_assert(NT == 1, "one row tile");
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc[0][ct]) : "v"(vop), "v"(p[0][ks]));
+__device__ __forceinline__ void wpv_step(f32x16_t &acc, bf16x8_t vop, const u32x4_t &p) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(vop), "v"(p));
 }
 // Zeroes one accumulator tile with an MFMA on zero operands: as an assignment of zeros, the compiler kept one tile's
 // zeros in scratch across the restart loop at head 512 (all 256 AGPRs hold accumulators there). Only PV MFMAs, which
@@ -264,13 +246,11 @@ __device__ __forceinline__ void wzero(f32x16_t &acc) {
 // 24 wait states: the last inline 32x32x16 MFMA's result (16 passes) is complete before anything else touches it
 __device__ __forceinline__ void wpv_drain() { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory"); }
 
-template <int HS, int KFMT, bool SPAN, bool BS16>
+template <bool SPAN, bool BS16>
 __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const PrefillParams p) {
-  using Sh = WShape<HS, KFMT>;
-  using Pf = PfShape<HS, KFMT>;
-  using St = WStager<HS, KFMT>;
-  constexpr int NT = wide_nt<HS>();
-  constexpr int kRowsWave = 32 * NT;
+  using Sh = WShape;
+  using St = WStager;
+  constexpr int kRowsWave = 32;
   constexpr int kRows = kPfWaves * kRowsWave;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[Sh::kLds];
   __shared__ int restart_word;
@@ -306,7 +286,7 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
   const int ke = uniform(min(kend, kb + seg));
   if (S > 1 && kb >= n) return;  // inactive segment: the merge does not read it
 
-  // ---- the wave's rows: tile jt, lane row col -> local row r0 + 32 (NT w + jt) + col = (token, head j)
+  // ---- the wave's rows: lane row col -> local row r0 + 32 w + col = (token, head j)
   // With rotation signs, the wave first rotates its rows into LDS (before any copy uses it): row by row with all 64
   // lanes (HS / 64 channels each), x D then the Walsh-Hadamard butterflies in ascending channel-bit order, as the
   // separate rotation pass does, then one bf16 rounding; the operands then load from there.
@@ -337,39 +317,35 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
     }
     wave_sync();
   }
-  WRows<HS, NT> r;
+  WRows r;
+  const int rr = r0 + kRowsWave * w + col;
+  const bool rv = rr < nrows;
+  const int tok = rv ? rr / G : 0, jh = rv ? rr % G : 0;
+  r.row_pos = rv ? n - qlen + tok : 0x3FFFFFFF;
+  const uint16_t *qr = p.qsigns ? nullptr : p.q + (int64_t)(q0 + tok) * p.qs0 + (int64_t)(kvh * G + jh) * p.qs1;
+  const uint16_t *qs_row = qrot + col * HS;
+  float qs = 0.f;  // the row's query sum: the 128 offset of the key operands (and the int4 zero point) folds into it
+  // the lane's channels: step_chan(cs, h) + e, e = 0..7, for cs = 0 .. HS / 16 - 1
 #pragma unroll
-  for (int jt = 0; jt < NT; ++jt) {
-    const int rr = r0 + kRowsWave * w + 32 * jt + col;
-    const bool rv = rr < nrows;
-    const int tok = rv ? rr / G : 0, jh = rv ? rr % G : 0;
-    r.row_pos[jt] = rv ? n - qlen + tok : 0x3FFFFFFF;
-    r.valid[jt] = rv;
-    const uint16_t *qr = p.qsigns ? nullptr : p.q + (int64_t)(q0 + tok) * p.qs0 + (int64_t)(kvh * G + jh) * p.qs1;
-    const uint16_t *qs_row = qrot + (32 * jt + col) * HS;
-    float qs = 0.f;  // the row's query sum: the 128 offset of the key operands (and the int4 zero point) folds into it
-    // the lane's channels: step_chan(cs, h) + e, e = 0..7, for cs = 0 .. HS / 16 - 1
-#pragma unroll
-    for (int cs = 0; cs < HS / 16; ++cs) {
-      u32x4_t x;
-      if (p.qsigns) x = *reinterpret_cast<const u32x4_t *>(qs_row + Sh::step_chan(cs, h));
-      else x = rv ? *reinterpret_cast<const u32x4_t *>(qr + Sh::step_chan(cs, h)) : u32x4_t{0u, 0u, 0u, 0u};
-      qs += bf16_lo(x[0]) + bf16_hi(x[0]) + bf16_lo(x[1]) + bf16_hi(x[1]) + bf16_lo(x[2]) + bf16_hi(x[2]) +
-            bf16_lo(x[3]) + bf16_hi(x[3]);
-      u32x4_t y;  // K operand order per 8 channels: (c0, c4, c1, c5, c2, c6, c3, c7)
-      y[0] = (x[0] & 0xFFFFu) | (x[2] << 16);
-      y[1] = (x[0] >> 16) | (x[2] & 0xFFFF0000u);
-      y[2] = (x[1] & 0xFFFFu) | (x[3] << 16);
-      y[3] = (x[1] >> 16) | (x[3] & 0xFFFF0000u);
-      r.qop[jt][cs] = as_bf16x8(y);
-    }
-    qs += shfl_xor_f(qs, 32);
-    r.qsum[jt] = qs;
-    r.m[jt] = -INFINITY;
-    r.mnext[jt] = -INFINITY;
-    r.l[jt] = 0.f;  // (a split without tiles keeps these: its rows are written as empty)
-    r.c[jt] = 0.f;
+  for (int cs = 0; cs < HS / 16; ++cs) {
+    u32x4_t x;
+    if (p.qsigns) x = *reinterpret_cast<const u32x4_t *>(qs_row + Sh::step_chan(cs, h));
+    else x = rv ? *reinterpret_cast<const u32x4_t *>(qr + Sh::step_chan(cs, h)) : u32x4_t{0u, 0u, 0u, 0u};
+    qs += bf16_lo(x[0]) + bf16_hi(x[0]) + bf16_lo(x[1]) + bf16_hi(x[1]) + bf16_lo(x[2]) + bf16_hi(x[2]) +
+          bf16_lo(x[3]) + bf16_hi(x[3]);
+    u32x4_t y;  // K operand order per 8 channels: (c0, c4, c1, c5, c2, c6, c3, c7)
+    y[0] = (x[0] & 0xFFFFu) | (x[2] << 16);
+    y[1] = (x[0] >> 16) | (x[2] & 0xFFFF0000u);
+    y[2] = (x[1] & 0xFFFFu) | (x[3] << 16);
+    y[3] = (x[1] >> 16) | (x[3] & 0xFFFF0000u);
+    r.qop[cs] = as_bf16x8(y);
   }
+  qs += shfl_xor_f(qs, 32);
+  r.qsum = qs;
+  r.m = -INFINITY;
+  r.mnext = -INFINITY;
+  r.l = 0.f;  // (a split without tiles keeps these: its rows are written as empty)
+  r.c = 0.f;
   if (p.qsigns) __syncthreads();  // every wave holds its operands: the rotated rows' LDS is free for the copies
 
   const int32_t *trow = p.table + (int64_t)seq * p.table_stride;
@@ -412,24 +388,21 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
     return st;
   };
   // S^T of tile t: lane half h reads code dwords 32 h + cs of key col, two steps per 8-byte read
-  auto qk_tile = [&](f32x16_t (&sq)[NT], int t) {
+  auto qk_tile = [&](f32x16_t &sq, int t) {
     const uint8_t *kp = pk_of(t) + col * Sh::kCell + (HS / 4) * h;
 #pragma unroll
     for (int cs = 0; cs < HS / 16; ++cs)
-      wqk(sq[0], k_operand(reinterpret_cast<const u32x2_t *>(kp)[cs >> 1][cs & 1]), r.qop[0][cs], cs == 0,
+      wqk(sq, k_operand(reinterpret_cast<const u32x2_t *>(kp)[cs >> 1][cs & 1]), r.qop[cs], cs == 0,
           cs == HS / 16 - 1);
   };
   if (tid == 0) restart_word = 0;
 
   // One pass over the split's keys; a score beyond the headroom starts it again with the raised maxima.
   for (int pass = 0; ntiles > 0; ++pass) {
+    r.l = 0.f;
+    r.c = 0.f;
 #pragma unroll
-    for (int jt = 0; jt < NT; ++jt) {
-      r.l[jt] = 0.f;
-      r.c[jt] = 0.f;
-#pragma unroll
-      for (int ct = 0; ct < HS / 32; ++ct) wzero(r.acc[jt][ct]);
-    }
+    for (int ct = 0; ct < HS / 32; ++ct) wzero(r.acc[ct]);
     // ---- prologue: tiles 0..2 fetched, tile 0 and tile 1's scalars unpacked, tile 3 fetched, S(0), the first maximum,
     // P(0)
     fetch(0);
@@ -453,32 +426,29 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
       st.s_load();
       st.s_store();
     }
-    f32x16_t s[NT];
+    f32x16_t s;
     qk_tile(s, 0);
     if (pass == 0) {  // the running maximum starts kWideBias above the first tile's row maximum
       const uint8_t *sc = sc_of(0);
+      float mx = -INFINITY;
 #pragma unroll
-      for (int jt = 0; jt < NT; ++jt) {
-        float mx = -INFINITY;
+      for (int q = 0; q < 4; ++q) {
+        const float4 a4 = *reinterpret_cast<const float4 *>(sc + Sh::kScA + 4 * (8 * q + 4 * h));
+        const float4 e4 = *reinterpret_cast<const float4 *>(sc + Sh::kScE + 4 * (8 * q + 4 * h));
+        const float av[4] = {a4.x, a4.y, a4.z, a4.w}, ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float4 a4 = *reinterpret_cast<const float4 *>(sc + Sh::kScA + 4 * (8 * q + 4 * h));
-          const float4 e4 = *reinterpret_cast<const float4 *>(sc + Sh::kScE + 4 * (8 * q + 4 * h));
-          const float av[4] = {a4.x, a4.y, a4.z, a4.w}, ev[4] = {e4.x, e4.y, e4.z, e4.w};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            float v = fmaf(s[jt][4 * q + j], av[j], -(r.qsum[jt] * ev[j]));
-            const int key = tile_key(0) + 8 * q + 4 * h + j;
-            if (key > r.row_pos[jt] || key >= ke) v = -INFINITY;
-            mx = fmaxf(mx, v);
-          }
+        for (int j = 0; j < 4; ++j) {
+          float v = fmaf(s[4 * q + j], av[j], -(r.qsum * ev[j]));
+          const int key = tile_key(0) + 8 * q + 4 * h + j;
+          if (key > r.row_pos || key >= ke) v = -INFINITY;
+          mx = fmaxf(mx, v);
         }
-        mx = fmaxf(mx, shfl_xor_f(mx, 32));
-        r.m[jt] = mx == -INFINITY ? mx : mx + kWideBias;
       }
+      mx = fmaxf(mx, shfl_xor_f(mx, 32));
+      r.m = mx == -INFINITY ? mx : mx + kWideBias;
     }
-    u32x4_t pop[NT][2];
-    if (w_softmax<HS, KFMT, NT, true>(r, s, sc_of(0), tile_key(0), ke, pop, lane)) restart_word = 1;
+    u32x4_t pop[2];
+    if (w_softmax<true>(r, s, sc_of(0), tile_key(0), ke, pop, lane)) restart_word = 1;
 
     // block ids of tile 4 onwards, a tile ahead of their copies, through the scalar cache
     const __attribute__((address_space(4))) int32_t *ctab = (const __attribute__((address_space(4))) int32_t *)trow;
@@ -524,7 +494,7 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
       // ---- phase A: S^T of tile it + 1 beside the unpack of its V and of tile it + 2's scalars; past the last tiles a
       // stale slot goes into idle buffers, the same code path
       St st = stager(it + 1, it + 2, kSteady);
-      f32x16_t sn[NT];
+      f32x16_t sn;
       const uint8_t *kp = pk_of(it + 1) + col * Sh::kCell + (HS / 4) * h;
       constexpr int kCs = HS / 16;
       u32x2_t kraw[2];  // code dword pairs j (steps 2 j, 2 j + 1) at kraw[j & 1], read two pairs ahead
@@ -535,7 +505,7 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
         const uint32_t x = kraw[(cs >> 1) & 1][cs & 1];
         if ((cs & 1) && (cs >> 1) + 2 < kCs / 2)
           kraw[(cs >> 1) & 1] = *reinterpret_cast<const u32x2_t *>(kp + 8 * ((cs >> 1) + 2));
-        wqk(sn[0], k_operand(x), r.qop[0][cs], cs == 0, cs == kCs - 1);
+        wqk(sn, k_operand(x), r.qop[cs], cs == 0, cs == kCs - 1);
         // the unpack, spread over the steps: the V units, then the scalars
 #pragma unroll
         for (int j = 0; j < St::kVUnits; ++j) {
@@ -550,7 +520,7 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
         if (cs == 4 + 8 * St::kVUnits) st.s_store();
       }
       // ---- phase B: O^T += V^T P^T of tile it beside the softmax of tile it + 1
-      u32x4_t pn[NT][2];
+      u32x4_t pn[2];
       bool over = false;
       {
         const uint8_t *vr = vb_of(it) + col * Sh::kVtRow + 16 * h;
@@ -566,16 +536,13 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
             const int nt = (sidx + 2) >> 1, nk = (sidx + 2) & 1;
             vbuf[sidx & 1] = *reinterpret_cast<const bf16x8_t *>(vr + 32 * Sh::kVtRow * nt + 32 * nk);
           }
-          wpv_step<NT>(r.acc, ct, vop, pop, ks);
-          if (sidx == 1) over = w_softmax<HS, KFMT, NT, kMask>(r, sn, sc_of(it + 1), tile_key(it + 1), ke, pn, lane);
+          wpv_step(r.acc[ct], vop, pop[ks]);
+          if (sidx == 1) over = w_softmax<kMask>(r, sn, sc_of(it + 1), tile_key(it + 1), ke, pn, lane);
         }
       }
       if (__builtin_expect(over, 0)) restart_word = 1;
-#pragma unroll
-      for (int jt = 0; jt < NT; ++jt) {
-        pop[jt][0] = pn[jt][0];
-        pop[jt][1] = pn[jt][1];
-      }
+      pop[0] = pn[0];
+      pop[1] = pn[1];
     };
     const int nplain = min(ntiles, max(0, (vis_all - kb) / kPfKeys));  // tiles with every key visible to every row
     int it = 0;
@@ -593,15 +560,13 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
       for (int sidx = 0; sidx < 2 * (HS / 32); ++sidx) {
         const int ct = sidx >> 1, ks = sidx & 1;
         const bf16x8_t vop = *reinterpret_cast<const bf16x8_t *>(vr + 32 * Sh::kVtRow * ct + 32 * ks);
-        wpv_step<NT>(r.acc, ct, vop, pop, ks);
+        wpv_step(r.acc[ct], vop, pop[ks]);
       }
       break;
     }
     wpv_drain();
     // start again with the flagged rows' maxima raised
-#pragma unroll
-    for (int jt = 0; jt < NT; ++jt)
-      if (r.mnext[jt] > r.m[jt]) r.m[jt] = r.mnext[jt];
+    if (r.mnext > r.m) r.m = r.mnext;
     __syncthreads();
     if (tid == 0) restart_word = 0;
     __syncthreads();
@@ -610,48 +575,35 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_wide_kernel(const Prefi
   wpv_drain();
 
   // ---- epilogue: l and the zero-point sum over the two lane halves, store
+  const float l = r.l + shfl_xor_f(r.l, 32);
+  const float csum = r.c + shfl_xor_f(r.c, 32);
+  // (the kernel always runs split: the merge normalises and rotates the 512-channel rows)
+  if (!rv) return;
+  const int k = pf_partial_exponent(l);
+  auto scaled = [&](float v) { return __builtin_amdgcn_ldexpf(v - csum, -k); };
+  const int64_t row = q0 + tok, head = kvh * G + jh;
+  float *orow = p.so + row * p.sos0 + head * p.sos1 + (int64_t)split * HS;
 #pragma unroll
-  for (int jt = 0; jt < NT; ++jt) {
-    const float l = r.l[jt] + shfl_xor_f(r.l[jt], 32);
-    const float csum = r.c[jt] + shfl_xor_f(r.c[jt], 32);
-    const bool valid = r.valid[jt];
-    const int rr = r0 + kRowsWave * w + 32 * jt + col;
-    const int64_t tok = q0 + (valid ? rr / G : 0);
-    const int64_t head = kvh * G + (valid ? rr % G : 0);
-    // (the kernel always runs split: the merge normalises and rotates the 512-channel rows)
-    if (valid) {
-      const int k = pf_partial_exponent(l);
-      auto scaled = [&](float v) { return __builtin_amdgcn_ldexpf(v - csum, -k); };
-      float *orow = p.so + tok * p.sos0 + head * p.sos1 + (int64_t)split * HS;
+  for (int ct = 0; ct < HS / 32; ++ct)
 #pragma unroll
-      for (int ct = 0; ct < HS / 32; ++ct)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x16_t &a = r.acc[jt][ct];
-          *reinterpret_cast<float4 *>(orow + 32 * ct + 8 * q + 4 * h) =
-              make_float4(scaled(a[4 * q]), scaled(a[4 * q + 1]), scaled(a[4 * q + 2]), scaled(a[4 * q + 3]));
-        }
-      if (h == 0) {
-        const int64_t st = tok * p.sts0 + head * p.sts1 + split;
-        p.smax[st] = r.m[jt] + (float)k;
-        p.ssum[st] = __builtin_amdgcn_ldexpf(l, -k);
-      }
+    for (int q = 0; q < 4; ++q) {
+      const f32x16_t &a = r.acc[ct];
+      *reinterpret_cast<float4 *>(orow + 32 * ct + 8 * q + 4 * h) =
+          make_float4(scaled(a[4 * q]), scaled(a[4 * q + 1]), scaled(a[4 * q + 2]), scaled(a[4 * q + 3]));
     }
+  if (h == 0) {
+    const int64_t st = row * p.sts0 + head * p.sts1 + split;
+    p.smax[st] = r.m + (float)k;
+    p.ssum[st] = __builtin_amdgcn_ldexpf(l, -k);
   }
 }
 
-template <int HS, int KFMT>
-void launch_wide(const PrefillParams &p, dim3 grid, bool span, hipStream_t s) {
-  if (span && p.block_size == 16) prefill_wide_kernel<HS, KFMT, true, true><<<grid, kPfWaves * 64, 0, s>>>(p);
-  else if (span) prefill_wide_kernel<HS, KFMT, true, false><<<grid, kPfWaves * 64, 0, s>>>(p);
-  else prefill_wide_kernel<HS, KFMT, false, false><<<grid, kPfWaves * 64, 0, s>>>(p);
-}
+int prefill_wide_rows() { return kPfWaves * 32; }
 
-int prefill_wide_rows() { return kPfWaves * 32 * wide_nt<512>(); }
-
-// Head 512 with int4 keys.
 void prefill_wide(const PrefillParams &p, dim3 grid, bool span, hipStream_t s) {
-  launch_wide<512, QP_CODES_INT4>(p, grid, span, s);
+  if (span && p.block_size == 16) prefill_wide_kernel<true, true><<<grid, kPfWaves * 64, 0, s>>>(p);
+  else if (span) prefill_wide_kernel<true, false><<<grid, kPfWaves * 64, 0, s>>>(p);
+  else prefill_wide_kernel<false, false><<<grid, kPfWaves * 64, 0, s>>>(p);
 }
 
 }  // namespace qp
