@@ -10,8 +10,8 @@
 //     them in token groups and the merge writes their output;
 //   * every other sequence takes the MFMA prefill kernel (or its query-slice path), which skips the short ones.
 // One longer sequence alone goes to the prefill kernel without a table.
-// A batch with short sequences only keeps the tokens' own rows and no table, so it needs no workspace and can be
-// recorded in a HIP graph. The randomized Hadamard rotation is fused: the kernels rotate each query row as it loads
+// A batch with short sequences only keeps the tokens' own rows and no table; where the segment buffers hold those rows it
+// needs no workspace and can be recorded in a HIP graph as it is. The randomized Hadamard rotation is fused: the kernels rotate each query row as it loads
 // and the merge / the prefill epilogue rotate the output back before the one bf16 store.
 #include "qp_common.h"
 
@@ -20,8 +20,9 @@
 
 namespace qp {
 
-// One workgroup. route_row[i]: first segment-buffer row of short sequence i, -1 for the others. row_tok / row_seq[r]: token and sequence of row r,
-// -1 / 0 for unused rows.
+// One workgroup. route_row[i]: first segment-buffer row of short sequence i, -1 for the others. row_tok / row_seq[r]: token
+// and sequence of row r, -1 / 0 for unused rows. rows_cap holds every short sequence's rows as long as q has the rows that
+// cu_q covers; a sequence past it is left to the prefill rather than written past the table.
 __global__ __launch_bounds__(256) void route_kernel(const int32_t *cu_q, int num_seqs, int rows_cap,
                                                     int32_t *route_row, int32_t *row_tok, int32_t *row_seq) {
   __shared__ int scan[256];
@@ -140,7 +141,9 @@ AttentionPlan plan_attention(const qp_paged_cache *cache, const qp_attention_arg
                    a->max_query_len * G <= 32 && a->num_tokens <= std::max<int64_t>(a->segm_rows, cap);
   // A single sequence of more than QP_DECODE_MAX_QUERY tokens needs no table to go to the prefill kernel: the route kernel
   // and the decode and merge launches that find nothing to do took 10 us of 55 (512 tokens of 32 heads of 64 over 4096).
-  const bool tables = decode_shape && !P.plain_decode;  // the workspace has the sequences' table, used or not
+  // The workspace has the sequences' table, used or not: a batch with longer sequences always asks for one, which tells it
+  // from a decode step (DecodePlan, qp_attention_noalloc), and a call without one stays refused.
+  const bool tables = decode_shape && !P.plain_decode;
   P.one_chunk = tables && a->num_seqs == 1 && a->num_tokens > QP_DECODE_MAX_QUERY &&
                 a->max_query_len > QP_DECODE_MAX_QUERY;
   P.routed = tables && !P.one_chunk;

@@ -164,7 +164,7 @@ struct PfStager {
       *reinterpret_cast<u32x2_t *>(kd + kk * Sh::kKdRow + 16 * Sh::kd_unit(d >> 1) + 8 * (d & 1)) = i8_quad_bf16(x);
     }
   }
-  // V unit (q4, ko) = tid mod HS (with HS = 128 the upper half repeats the lower half's unit: same bytes, same place)
+  // V unit (q4, ko) of the thread
   __device__ __forceinline__ int vunit() const { return tid & (HS - 1); }
   __device__ __forceinline__ void v_load(int s) {
     const int u = vunit(), ko = u & 3, q4 = u >> 2;

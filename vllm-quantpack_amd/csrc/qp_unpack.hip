@@ -129,7 +129,7 @@ extern "C" int qp_unpack_segment(const qp_cache_half *half, int32_t block_size, 
                        ? (out_stride[0] % 8 == 0 && out_stride[1] % 8 == 0 && ((uintptr_t)out & 15) == 0)
                        : (out_stride[0] % 4 == 0 && out_stride[1] % 4 == 0 && ((uintptr_t)out & 7) == 0);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // launches of fewer than 2^31 dwords (one, unless the segment's output is past 16 GiB)
+  // launches of at most 2^30 dwords of codes (one, unless the output is past 16 GiB, or 8 GiB of int8 keys)
   const int64_t per_token = (int64_t)num_kv_heads * p.dw;
   QP_SUPPORTED(per_token < (int64_t(1) << 30), "qp_unpack_segment: rows of a token too large");
   const int64_t most = (int64_t(1) << 30) / per_token;
