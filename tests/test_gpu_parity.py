@@ -690,8 +690,8 @@ def test_prefill_repeats_bit_for_bit(device, fmt, splits, hs, nq, nkv):
     waves (a copy landing in a slot that is still read, an LDS buffer rewritten before a barrier) or a work split that
     follows the waves' timing shows up here as differing rows, well inside the accuracy bars the other tests hold.
     40 tokens over 3000 keys: at head 256 (6 query heads per KV head) two row blocks of the tile kernel through its
-    unrolled and steady loops; head 128 with 8 per KV head and head 512 on the wide kernel; head 512 with int8 keys as
-    query slices on the decode kernel; one split, or the host's choice (split partials merged)."""
+    unrolled and steady loops; head 128 with 8 per KV head on the dual kernel; head 512 on the wide kernel, with int8 keys
+    as query slices on the decode kernel; one split, or the host's choice (split partials merged)."""
     import torch
 
     from vllm_quantpack.attention import int4_prefill
@@ -816,8 +816,7 @@ def test_prefill_head_512(device, fmt):
 
 @pytest.mark.parametrize("fmt", ["int4", "int8"])
 def test_prefill_head_64(device, fmt):
-    """Head 64 prefills over causal query slices of the split-KV kernel (the reference's kernels take any head size:
-    int4_kv.py:130-131). Ragged batch, with a first chunk (context == chunk)."""
+    """Head 64 prefills on the dual kernel (the reference's kernels take any head size: int4_kv.py:130-131). Ragged batch, with a first chunk (context == chunk)."""
     rng = np.random.default_rng(407 + (1 if fmt == "int8" else 0))
     out, emu, ref = _prefill_case(device, rng, fmt, [(37, 2100), (20, 20), (1, 64)], nq=16, nkv=2, hs=64)
     assert_emulation(out, emu)
@@ -838,8 +837,7 @@ def test_prefill_tile_rows_at_any_gqa_width(device, nq, nkv, hs):
 
 
 def test_prefill_wide_gqa(device):
-    """16 query heads per KV head is past the 16-row-tile kernel's 12: the wide kernel (32x32x16 MFMAs, rows as
-    (token, head) pairs) serves it."""
+    """16 query heads per KV head at head 128, on the dual kernel (32x32x16 MFMAs, rows as (token, head) pairs)."""
     rng = np.random.default_rng(405)
     out, emu, ref = _prefill_case(device, rng, "int4", [(20, 1500), (3, 200)], nq=16, nkv=1, hs=128)
     assert_emulation(out, emu)
@@ -849,8 +847,8 @@ def test_prefill_wide_gqa(device):
 @pytest.mark.parametrize("fmt", ["int4", "int8"])
 @pytest.mark.parametrize("hs,splits", [(256, 1), (256, 3), (128, 1), (128, 2), (512, 1), (512, 3)])
 def test_prefill_wide_kernel_batches(device, fmt, hs, splits):
-    """16 query heads per KV head on a batch whose row blocks (256 rows at head 128 and 128 at head 512 on the wide
-    kernel, 192 at head 256 on the tile kernel) straddle tokens and end mid-block: a long chunk, a first chunk (context
+    """16 query heads per KV head on a batch whose row blocks (256 rows at head 128 on the dual kernel, 128 at head 512
+    on the wide kernel, 192 at head 256 on the tile kernel) straddle tokens and end mid-block: a long chunk, a first chunk (context
     == chunk), a single token, a 130-token chunk; 32 query heads on 2 KV heads; with key splits, some of them empty
     (head 512 runs at least 2; with int8 keys it takes the query slices)."""
     rng = np.random.default_rng(260 + hs + splits + (1 if fmt == "int8" else 0))
@@ -864,7 +862,7 @@ def test_prefill_wide_kernel_batches(device, fmt, hs, splits):
 @pytest.mark.parametrize("fmt,n,hs", [("int4", 330, 128), ("int8", 1000, 128), ("int4", 1009, 512), ("int4", 353, 512)])
 def test_prefill_wide_table_row_exactly_as_long_as_the_context(device, fmt, n, hs):
     """One sequence whose block table holds exactly ceil(n / 16) entries and whose last tile has 1..16 keys, on the
-    wide kernel (the CPU walk in test_prefill_table_walk checks its table reads)."""
+    dual kernel (head 128) and the wide one (the CPU walk in test_prefill_table_walk checks its table reads)."""
     rng = np.random.default_rng(270 + n)
     out, emu, ref = _prefill_case(device, rng, fmt, [(20, n)], nq=16, nkv=1, hs=hs)
     assert_emulation(out, emu)
@@ -874,8 +872,8 @@ def test_prefill_wide_table_row_exactly_as_long_as_the_context(device, fmt, n, h
 @pytest.mark.parametrize("hs", [128, 256, 512])
 def test_prefill_wide_rows_without_keys_are_zero(device, hs):
     """A sequence whose context holds no keys (seqused_k = 0 beside a query chunk; vLLM does not send these) leaves
-    the row blocks without a tile (the wide kernel at heads 128 and 512, the tile kernel at 256): its rows come out
-    zero, with one split (the epilogue's normalisation of empty accumulators) and with several (every split empty for
+    the row blocks without a tile (the dual kernel at head 128, the tile kernel at 256, the wide one at 512): its rows come
+    out zero, with one split (the epilogue's normalisation of empty accumulators) and with several (every split empty for
     the merge), and the other sequence is unaffected."""
     import torch
 
@@ -905,8 +903,8 @@ def test_prefill_wide_rows_without_keys_are_zero(device, hs):
 @pytest.mark.parametrize("fmt,hs", [("int4", 128), ("int8", 128), ("int4", 512)])
 def test_prefill_wide_scores_far_above_the_first_tile(device, fmt, hs):
     """Key scales of 2^7 .. 2^12 late in the context put scores thousands of log2 units above the first tile's
-    maximum, past the wide kernel's headroom: the workgroup runs its split again with the raised maxima (once per
-    jump), and the result still matches."""
+    maximum, past the headroom of the dual kernel (head 128) and the wide one: the workgroup runs its split again with the
+    raised maxima (on the wide kernel once per jump), and the result still matches."""
     rng = np.random.default_rng(280 + (1 if fmt == "int8" else 0) + hs)
     big = [(700, 2.0 ** 7), (1300, 2.0 ** 9), (1901, 2.0 ** 12)]
     out, emu, ref = _prefill_case(device, rng, fmt, [(40, 2000), (9, 1400)], nq=16, nkv=1, hs=hs, splits=1,
@@ -917,7 +915,7 @@ def test_prefill_wide_scores_far_above_the_first_tile(device, fmt, hs):
 
 @pytest.mark.parametrize("hs", [128, 512])
 def test_prefill_wide_fused_rotations(device, hs):
-    """On the wide kernel: the query rotated on load gives the bits of rotating it first, and the output rotated back
+    """On the dual kernel (head 128) and the wide one: the query rotated on load gives the bits of rotating it first, and the output rotated back
     in the epilogue (one split) or by the merge (three; at head 512 the kernel always splits) matches a separate
     inverse rotation."""
     import torch
@@ -950,8 +948,8 @@ def test_prefill_wide_fused_rotations(device, hs):
 
 @pytest.mark.parametrize("fmt,hs,nq", [("int8", 256, NQ), ("int4", 512, 16), ("int8", 128, 16)])
 def test_prefill_span_and_row_loaders_agree(device, fmt, hs, nq):
-    """The page-run copies (HND) and the strided gather (NHD) of the tile kernel (head 256) and the wide one (head 128
-    with 8 query heads per KV head, head 512) on the same cache contents."""
+    """The page-run copies (HND) and the strided gather (NHD) of the tile kernel (head 256), the wide one (head 512)
+    and the dual one (head 128) on the same cache contents."""
     case = dict(hs=hs, nq=nq, nkv=2 if hs in (128, 512) else NKV)
     a, emu, ref = _prefill_case(device, np.random.default_rng(204), fmt, [(64, 1500), (3, 700)], **case)
     b, _, _ = _prefill_case(device, np.random.default_rng(204), fmt, [(64, 1500), (3, 700)], layout="nhd", **case)

@@ -49,3 +49,15 @@ def test_splits_whose_maxima_rise_after_their_first_keys(device, fmt, hs, G, ord
     out, ref = _attend(device, fmt, hs, scores, 7, G, 3, 40 + hs)
     assert np.isfinite(out).all()
     assert O.relerr(out, ref) < 5e-3, O.relerr(out, ref)
+
+
+@pytest.mark.parametrize("fmt,hs,G", [("int4", 64, 4), ("int8", 64, 4), ("int4", 128, 4), ("int8", 128, 8), ("int4", 512, 4)])
+def test_splits_that_run_again_beside_others(device, fmt, hs, G):
+    """Two splits whose later keys score 250 to 300 above their first (past the headroom, so their workgroups start again
+    with the true maxima) and one that is high from its first key on and does not."""
+    a = np.concatenate((np.full(100, 1.0), [300.0], np.full(923, 2.0)))
+    b = np.concatenate((np.full(32, 3.0), np.full(492, 251.0), np.full(500, 291.0)))
+    c = np.concatenate((np.full(40, 292.0), np.full(984, 280.0)))
+    out, ref = _attend(device, fmt, hs, np.concatenate((a, b, c)), 5, G, 3, 60 + hs)
+    assert np.isfinite(out).all()
+    assert O.relerr(out, ref) < 5e-3, O.relerr(out, ref)

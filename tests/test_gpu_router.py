@@ -114,7 +114,7 @@ def test_mixed_batch_long_prefill_and_mtp_decodes(device, fmt):
 
 @pytest.mark.parametrize("fmt", ["int4", "int8"])
 def test_mixed_batch_head_64(device, fmt):
-    """Head 64 through the drop-in: a 40-token chunk (query slices of the split-KV kernel) beside decodes of 4 and 1
+    """Head 64 through the drop-in: a 40-token chunk (the dual prefill kernel) beside decodes of 4 and 1
     tokens, the rotations fused, 16 query heads on 2 KV heads; within 0.5 % of fp64."""
     import torch
     seqs = [(40, 3000), (4, 2000), (1, 700)]
