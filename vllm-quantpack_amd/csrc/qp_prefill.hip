@@ -903,10 +903,10 @@ constexpr int kMinSplitKeys = 1024;
 
 // Which kernel serves a prefill:
 //   * heads 64 and 128: the dual kernel (qp_prefill_dual.hip), two waves per SIMD, at every GQA width and chunk length.
-//     2048 tokens over 16384 keys with 64 q / 8 KV heads of 128: 1.22-1.31 ms against 1.96 on the wide kernel's 32x32x16
-//     MFMAs with one wave per SIMD; 8 prompts of up to 2048 tokens with 32 q / 8 KV heads: 147 against 265 us on four
-//     16-row tiles per wave of the tile kernel; 512 tokens over 4096 keys with 32 q / 8 KV heads of 64: 58 against 94 us
-//     as query slices;
+//     2048 tokens over 16384 keys with 64 q / 8 KV heads of 128: 1.25-1.29 ms against 1.96 on 32x32x16 MFMAs with one
+//     wave per SIMD; 8 prompts of up to 2048 tokens with 32 q / 8 KV heads: 146 against 265 us on four 16-row tiles per
+//     wave of the tile kernel; 512 tokens over 4096 keys with 32 q / 8 KV heads of 64: 48-49 against 94 us as query
+//     slices;
 //   * head 256, whose accumulators and query operands leave room for one wave per SIMD: the tile kernel above, whose
 //     192-row blocks hold (token, head) pairs at any GQA width. With 16 heads per KV head it takes 1.63 ms against
 //     1.72 on 32x32x16 MFMAs (one 32-row tile per wave there: each K / V operand read from LDS serves 32 rows against

@@ -13,7 +13,8 @@
 // key split; a tile of 64 keys is unpacked once for all rows, with one barrier per tile.
 //   * 32x32x16 MFMAs: with two waves per SIMD (a loop of MFMAs with N independent FMAs after each, both waves running it)
 //     the SIMD takes about max(32, 11 + 4 N) cycles per 32x32x16 MFMA and max(16, 9 + 4 N) per 16x16x32 one, and this
-//     kernel has about 6 VALU instructions per 32x32x16 MFMA, so the larger shape hides nearly all of them.
+//     kernel has 6.2 VALU instructions per 32x32x16 MFMA at head 128 folded and 7.9 otherwise, so the larger shape hides
+//     most of them.
 //   * The tile's packed pages are copied HBM -> LDS four tiles ahead (global_load_lds_dwordx4, one or two copies per
 //     wave). Past the end of the split the last run is copied again, so no iteration has an end case.
 //   * A tile is worked through in 32-key sub-tiles u: the MFMAs of S^T = K Q^T of sub-tile u + 1 and of O^T += V^T P^T of
@@ -27,14 +28,15 @@
 // two nibbles of a code byte): a thread's stores then go to two runs of whole rows, and a lane's accumulators hold 8
 // consecutive output channels.
 //
-// What bounds it, and what it measured (64 q / 8 KV heads of 128, 2048 tokens over 16384 cached keys, int4): 1.22-1.31 ms
-// = 890-960 TFLOP/s against 1.96 ms on 32x32x16 MFMAs with one wave per SIMD; MFMAs busy 48 % of the cycles at about 2.1
-// GHz (2.3 GHz under the head-256 kernel: this one draws more power), the LDS active 55 %. Without the softmax 1.04 ms,
-// without the unpack 1.10 ms, without both, the copies and the operand re-reads 0.79 ms. The order of the steps hardly
-// matters: reads two sub-tiles ahead, fences between the steps, raised wave priorities and the build's scheduler are all
-// within 2 %. 16x16x32 MFMAs with the phases in turn took 1.27 ms, the two halves of the waves half a tile apart behind
-// a barrier per half 1.45 ms. 8 prompts of 128..2048 tokens, 32 q / 8 KV heads: 147 against 265 us on four 16-row tiles
-// per wave; head 64 (32 q / 8 KV heads, 512 tokens over 4096, int8 keys): 58-60 against 94 us as query slices.
+// What bounds it, and what it measured (64 q / 8 KV heads of 128, 2048 tokens over 16384 cached keys, int4): 1.25-1.29 ms
+// = 909-935 TFLOP/s (1.46 ms on the slowest box) against 1.96 ms on 32x32x16 MFMAs with one wave per SIMD; MFMAs busy 46 %
+// of the cycles at about 2.1 GHz (2.3 GHz under the head-256 kernel: this one draws more power), the LDS active 53 %. The
+// following were measured on the folded form (1.21 ms): without the softmax 1.04 ms, without the unpack 1.10 ms, without
+// both, the copies and the operand re-reads 0.79 ms. The order of the steps hardly matters: reads two sub-tiles ahead,
+// fences between the steps, raised wave priorities and the build's scheduler are all within 2 %. 16x16x32 MFMAs with the
+// phases in turn took 1.27 ms, the two halves of the waves half a tile apart behind a barrier per half 1.45 ms. 8 prompts
+// of 128..2048 tokens, 32 q / 8 KV heads: 146 against 265 us on four 16-row tiles per wave; head 64 (32 q / 8 KV heads,
+// 512 tokens over 4096, int8 keys): 48-49 against 94 us as query slices.
 #include "qp_prefill.h"
 
 #include <type_traits>
@@ -136,10 +138,11 @@ __host__ __device__ __forceinline__ uint32_t dual_share(uint32_t pairs) {
 // FOLD: the value scales are folded into the scores (the QK accumulators start at b = log2(s_v) / a, so one exp2 gives
 // P s_v) and l comes out of the zero-point tile's MFMA, as in the head-256 tile kernel; it normalises by the rounded
 // weights, and a key whose value scale is 0 drops out of it. Otherwise l is summed in fp32 from the unrounded P, two VALU
-// instructions more per score. Each shape keeps the form that it has always had (dual_folds): 8 prompts of up to 2048
-// tokens, 32 q / 8 KV heads of 128: 155 us and 2.7e-3 off the 64-bit result folded, 160 us and 3.0e-3 otherwise; 2048
-// tokens over 16384 keys, 64 q / 8 KV heads: 1409 us and 3.7e-3, 1463 us and 3.8e-3; 512 tokens over 4096, 32 q / 8 KV
-// heads of 64: 48.4 us and 3.5e-3, 51.2 us and 3.6e-3.
+// instructions more per score. A shape has the form of the kernel that served it before this one, so that its sums keep
+// their bits (dual_folds: the tile kernel folds, the query slices and 32x32x16 MFMAs with one wave per SIMD did not). Both
+// forms, on one box, and how far they are off the 64-bit result: 8 prompts of up to 2048 tokens, 32 q / 8 KV heads of 128: 155 us and 2.7e-3 folded, 160 us and 3.0e-3 otherwise;
+// 2048 tokens over 16384 keys, 64 q / 8 KV heads: 1409 us and 3.7e-3, 1463 us and 3.8e-3; 512 tokens over 4096, 32 q / 8
+// KV heads of 64: 48.4 us and 3.5e-3, 51.2 us and 3.6e-3.
 template <int HS, int KFMT, bool SPAN, bool FOLD>
 __global__ __launch_bounds__(kDualThreads) void prefill_dual_kernel(const PrefillParams p) {
   using Sh = DualShape<HS, KFMT>;
